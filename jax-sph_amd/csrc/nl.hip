@@ -111,6 +111,13 @@ __device__ __forceinline__ int wave_run_slot(int32_t* __restrict__ counter, int 
   return __shfl(base, first, 64) + lane - first;
 }
 
+// Start of a build: the bits of the list before (sticky), the rest zero.
+__device__ __forceinline__ void reset_info(int64_t* __restrict__ info,
+                                           const int64_t* __restrict__ prev) {
+  info[0] = prev ? prev[0] : 0;
+  for (int k = 1; k < 8; ++k) info[k] = 0;
+}
+
 template <int DIM>
 __device__ __forceinline__ void hash_count_body(const float* __restrict__ r, int n, const Grid& g,
                                                 int32_t* __restrict__ cell_count,
@@ -137,7 +144,10 @@ __device__ __forceinline__ void hash_count_body(const float* __restrict__ r, int
 template <int DIM>
 __global__ void k_hash_count(const float* __restrict__ r, int n, Grid g,
                              int32_t* __restrict__ cell_count, int32_t* __restrict__ pcell,
-                             int32_t* __restrict__ pslot, const int32_t* __restrict__ gate) {
+                             int32_t* __restrict__ pslot, const int32_t* __restrict__ gate,
+                             int64_t* __restrict__ info = nullptr,
+                             const int64_t* __restrict__ prev = nullptr) {
+  if (info && blockIdx.x == 0 && threadIdx.x == 0) reset_info(info, prev);
   hash_count_body<DIM>(r, n, g, cell_count, pcell, pslot, gate, blockIdx.x);
 }
 
@@ -218,7 +228,9 @@ __global__ __launch_bounds__(kBlock) void k_integrate_hash(
     const float* __restrict__ r, const float* __restrict__ u, const float* __restrict__ dudt,
     const float* __restrict__ dvdt, float* __restrict__ r_out, float* __restrict__ u_out,
     float* __restrict__ v_out, int n, float dt, float ctvf, Grid g, float bx, float by, float bz,
-    int32_t* __restrict__ cell_count, int32_t* __restrict__ pcell, int32_t* __restrict__ pslot) {
+    int32_t* __restrict__ cell_count, int32_t* __restrict__ pcell, int32_t* __restrict__ pslot,
+    int64_t* __restrict__ info, const int64_t* __restrict__ prev) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) reset_info(info, prev);
   const float side[3] = {bx, by, bz};
   float x[3] = {0.f, 0.f, 0.f};
   const int i = integrate_block<DIM>(r, u, dudt, dvdt, r_out, u_out, v_out, n, dt, ctvf, side,
@@ -331,97 +343,169 @@ __global__ void k_max_reduce(const int32_t* __restrict__ a, int64_t n, int64_t* 
   if ((threadIdx.x & 63) == 0) atomicMax((unsigned long long*)out, (unsigned long long)m);
 }
 
-// Single-workgroup exclusive scan with wavefront (64-lane) inclusive scans.
-// out[k] = sum(in[0:k]) for k in [0, n]; also the max of in (for the cell capacity).
+// Exclusive scan: out[k] = sum(in[0:k]) for k in [0, n]; also the largest entry
+// (for the cell capacity).  Each workgroup scans `chunk` entries (a multiple of
+// kScanTile), four a thread and tile.  What precedes its chunk it adds up
+// itself: from the entries (they are in the L2 and no workgroup waits for
+// another) or, on long inputs, from the sums of the earlier chunks (SUMS).
 constexpr int kScanThreads = 1024;
-constexpr int kScanItems = 8;
+constexpr int kScanTile = 4 * kScanThreads;
+constexpr int kScanSums = 1024;  // chunk sums at most (sph_ws::scan_tmp)
 
-template <typename TIn, typename TOut>
-__device__ __forceinline__ void scan_single_body(const TIn* in, int64_t n, TOut* __restrict__ out,
-                                                 int64_t* __restrict__ max_out,
-                                                 int64_t* __restrict__ info, int64_t capacity,
-                                                 TIn* clear, const int32_t* __restrict__ gate) {
-  // `clear` (the input array itself, or null) is zeroed as it is read;
-  // `gate` (or null) skips the whole scan when *gate == 0.
-  __shared__ TOut wave_tot[kScanThreads / 64];
-  __shared__ TOut carry_s;
-  __shared__ int64_t wmax[kScanThreads / 64];
-  if (gate && *gate == 0) return;
-  const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
-  TOut carry = 0;
-  int64_t mx = 0;
-  const int64_t chunk = (int64_t)kScanThreads * kScanItems;
-  for (int64_t base = 0; base < n; base += chunk) {
-    TOut v[kScanItems];
-    TOut s = 0;
-    int64_t i0 = base + (int64_t)t * kScanItems;
+struct ScanPlan {
+  int64_t chunk;
+  int blocks;
+  bool sums;
+};
+// Adding up the entries costs a workgroup a load a thread for every chunk
+// before its own: 7.4 us for 30,300 entries (8 chunks; one workgroup, tile
+// after tile, took 37.5 us) and 15.8 us for 129,600 (32 chunks).  With the sums
+// both take 5.4 us, after another launch of 2.8 us and its gap: beyond 16
+// chunks that is the cheaper one.
+static ScanPlan scan_plan(int64_t n, bool have_sums) {
+  const int64_t tiles = n > 0 ? cdiv(n, kScanTile) : 1;
+  ScanPlan p;
+  p.chunk = kScanTile * cdiv(tiles, kScanSums);
+  p.blocks = (int)(n > 0 ? cdiv(n, p.chunk) : 1);
+  p.sums = have_sums && p.blocks > 16;
+  return p;
+}
+
+template <typename TIn>
+__device__ __forceinline__ void load4(const TIn* __restrict__ in, int64_t i, int64_t n, bool wide,
+                                      TIn* v) {
+  if (wide && i + 3 < n) {
+    const int4 q = *(const int4*)(in + i);
+    v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+  } else {
 #pragma unroll
-    for (int k = 0; k < kScanItems; ++k) {
-      int64_t i = i0 + k;
-      TOut x = i < n ? (TOut)in[i] : (TOut)0;
-      if (clear && i < n) clear[i] = 0;
-      v[k] = x;
-      s += x;
-      mx = (int64_t)x > mx ? (int64_t)x : mx;
-    }
-    // inclusive wave scan of the per-thread sums
-    TOut inc = s;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      TOut y = __shfl_up(inc, o, 64);
-      if (lane >= o) inc += y;
-    }
-    if (lane == 63) wave_tot[wid] = inc;
-    __syncthreads();
-    if (wid == 0) {
-      TOut w = lane < kScanThreads / 64 ? wave_tot[lane] : (TOut)0;
-      TOut winc = w;
-#pragma unroll
-      for (int o = 1; o < 16; o <<= 1) {
-        TOut y = __shfl_up(winc, o, 64);
-        if (lane >= o) winc += y;
-      }
-      if (lane < kScanThreads / 64) wave_tot[lane] = winc - w;  // exclusive
-      if (lane == kScanThreads / 64 - 1) carry_s = winc;
-    }
-    __syncthreads();
-    TOut run = carry + wave_tot[wid] + (inc - s);
-#pragma unroll
-    for (int k = 0; k < kScanItems; ++k) {
-      int64_t i = i0 + k;
-      if (i < n) out[i] = run;
-      run += v[k];
-    }
-    carry += carry_s;
-    __syncthreads();
-  }
-  // max reduction
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    int64_t y = __shfl_down(mx, o, 64);
-    mx = y > mx ? y : mx;
-  }
-  if (lane == 0) wmax[wid] = mx;
-  __syncthreads();
-  if (t == 0) {
-    out[n] = carry;
-    int64_t m = 0;
-    for (int w = 0; w < kScanThreads / 64; ++w) m = wmax[w] > m ? wmax[w] : m;
-    if (max_out) *max_out = m;
-    if (info && capacity >= 0 && m > capacity) info[0] |= SPH_CELL_LIST_OVERFLOW;
+    for (int k = 0; k < 4; ++k) v[k] = i + k < n ? in[i + k] : (TIn)0;
   }
 }
 
-template <typename TIn, typename TOut>
-__global__ __launch_bounds__(kScanThreads) void k_scan_single(const TIn* in, int64_t n,
-                                                              TOut* __restrict__ out,
-                                                              int64_t* __restrict__ max_out,
-                                                              int64_t* __restrict__ info,
-                                                              int64_t capacity,
-                                                              TIn* clear = nullptr,
-                                                              const int32_t* __restrict__ gate =
-                                                                  nullptr) {
-  scan_single_body<TIn, TOut>(in, n, out, max_out, info, capacity, clear, gate);
+// Sum over the workgroup, the same in every thread.
+template <typename T>
+__device__ __forceinline__ T block_sum(T x, T* part) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
+  __syncthreads();  // part may still be read from an earlier use
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = x;
+  __syncthreads();
+  T t = 0;
+#pragma unroll
+  for (int w = 0; w < kScanThreads / 64; ++w) t += part[w];
+  return t;
+}
+
+template <typename TOut>
+__global__ __launch_bounds__(kScanThreads) void k_chunk_sums(const int32_t* __restrict__ in,
+                                                             int64_t n, int64_t chunk,
+                                                             TOut* __restrict__ sums) {
+  __shared__ TOut part[kScanThreads / 64];
+  const int64_t lo = blockIdx.x * chunk, hi = lo + chunk < n ? lo + chunk : n;
+  const bool wide = ((uintptr_t)in & 15) == 0;
+  TOut s = 0;
+  for (int64_t i = lo + 4 * threadIdx.x; i < hi; i += kScanTile) {
+    int32_t v[4];
+    load4(in, i, n, wide, v);
+    s += (TOut)v[0] + v[1] + v[2] + v[3];
+  }
+  s = block_sum(s, part);
+  if (threadIdx.x == 0) sums[blockIdx.x] = s;
+}
+
+// blk, nblk: the workgroup's chunk and the chunks of this input.  With a gate,
+// runs only when *gate != 0; info (or null) receives the largest entry in
+// info[2] (zeroed before) and the cell-capacity bit.
+template <typename TOut>
+__device__ __forceinline__ void scan_body(const int32_t* __restrict__ in, int64_t n, int64_t chunk,
+                                          const TOut* __restrict__ sums, TOut* __restrict__ out,
+                                          int64_t* __restrict__ info, int64_t capacity,
+                                          const int32_t* __restrict__ gate, int blk, int nblk) {
+  __shared__ TOut part[kScanThreads / 64];
+  __shared__ int wmax[kScanThreads / 64];
+  if (gate && *gate == 0) return;  // uniform
+  const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
+  const bool wide = ((uintptr_t)in & 15) == 0;
+  const int64_t lo = blk * chunk, hi = lo + chunk < n ? lo + chunk : n;
+  TOut before = 0;
+  if (sums) {
+    for (int k = t; k < blk; k += kScanThreads) before += sums[k];
+  } else {
+    for (int64_t i = 4 * t; i < lo; i += kScanTile) {
+      int32_t v[4];
+      load4(in, i, n, wide, v);
+      before += (TOut)v[0] + v[1] + v[2] + v[3];
+    }
+  }
+  TOut carry = blk > 0 ? block_sum(before, part) : (TOut)0;
+  int mx = 0;
+  for (int64_t base = lo; base < hi; base += kScanTile) {
+    const int64_t i0 = base + 4 * t;
+    int32_t v[4];
+    load4(in, i0, n, wide, v);
+    const TOut s = (TOut)v[0] + v[1] + v[2] + v[3];
+    mx = max(max(mx, max(v[0], v[1])), max(v[2], v[3]));
+    TOut inc = s;  // inclusive scan over the wavefront
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const TOut y = __shfl_up(inc, o, 64);
+      if (lane >= o) inc += y;
+    }
+    __syncthreads();  // part of the tile before is no longer read
+    if (lane == 63) part[wid] = inc;
+    __syncthreads();
+    TOut run = carry + inc - s;
+    TOut tile = 0;
+#pragma unroll
+    for (int w = 0; w < kScanThreads / 64; ++w) {
+      const TOut x = part[w];
+      if (w < wid) run += x;
+      tile += x;
+    }
+    carry += tile;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if (i0 + k < n) out[i0 + k] = run;
+      run += v[k];
+    }
+  }
+  if (t == 0 && blk == nblk - 1) out[n] = carry;
+  if (!info) return;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) mx = max(mx, __shfl_down(mx, o, 64));
+  if (lane == 0) wmax[wid] = mx;
+  __syncthreads();
+  if (t == 0) {
+    int m = 0;
+    for (int w = 0; w < kScanThreads / 64; ++w) m = max(m, wmax[w]);
+    atomicMax((unsigned long long*)&info[2], (unsigned long long)m);
+    if (capacity >= 0 && m > capacity)
+      atomicOr((unsigned long long*)&info[0], (unsigned long long)SPH_CELL_LIST_OVERFLOW);
+  }
+}
+
+template <typename TOut>
+__global__ __launch_bounds__(kScanThreads) void k_scan(
+    const int32_t* __restrict__ in, int64_t n, int64_t chunk, const TOut* __restrict__ sums,
+    TOut* __restrict__ out, int64_t* __restrict__ info, int64_t capacity,
+    const int32_t* __restrict__ gate) {
+  scan_body<TOut>(in, n, chunk, sums, out, info, capacity, gate, blockIdx.x, gridDim.x);
+}
+
+// Scans in[0:n] into out[0:n + 1]; scratch (or null) holds kScanSums sums.
+template <typename TOut>
+static int scan(sph_ws* ws, const char* name, const int32_t* in, int64_t n, TOut* out,
+                TOut* scratch, int64_t* info, int64_t capacity, const int32_t* gate,
+                hipStream_t st) {
+  const ScanPlan p = scan_plan(n, scratch != nullptr);
+  if (p.sums)
+    SPH_LAUNCH(ws, "scan_sums", st,
+               k_chunk_sums<TOut><<<p.blocks, kScanThreads, 0, st>>>(in, n, p.chunk, scratch));
+  SPH_LAUNCH(ws, name, st,
+             k_scan<TOut><<<p.blocks, kScanThreads, 0, st>>>(
+                 in, n, p.chunk, p.sums ? scratch : nullptr, out, info, capacity, gate));
+  return SPH_OK;
 }
 
 __device__ __forceinline__ void scatter_body(const int32_t* __restrict__ pcell,
@@ -474,17 +558,20 @@ __device__ __forceinline__ unsigned long long cell_sort_key(int id, const float*
 // reference's stable argsort; with positions (skin lists, whose order is free)
 // the particles of a cell follow a Morton curve over its sub-cells, so that
 // consecutive particles, which share wavefronts in the sweeps, are close.
+// `clear` (or null): the cell histogram, zeroed here for the next binning.
 template <int DIM>
 __device__ __forceinline__ void cell_sort_body(const int32_t* __restrict__ cell_start,
                                                const int32_t* __restrict__ unsorted,
                                                int32_t* __restrict__ perm,
                                                int32_t* __restrict__ iperm, int64_t ncell,
                                                const int32_t* __restrict__ gate, int blk,
-                                               const float* __restrict__ r, const Grid& g) {
+                                               const float* __restrict__ r, const Grid& g,
+                                               int32_t* __restrict__ clear) {
   if (gate && *gate == 0) return;
   const int lane = threadIdx.x & 63;
   const int64_t cell = ((int64_t)blk * blockDim.x + threadIdx.x) >> 6;
   if (cell >= ncell) return;
+  if (clear && lane == 0) clear[cell] = 0;
   const int b = cell_start[cell], e = cell_start[cell + 1], n = e - b;
   if (n <= 64) {
     const unsigned long long key = lane < n ? cell_sort_key<DIM>(unsorted[b + lane], r, g)
@@ -517,8 +604,9 @@ __global__ __launch_bounds__(256) void k_cell_sort(const int32_t* __restrict__ c
                                                    int32_t* __restrict__ perm,
                                                    int32_t* __restrict__ iperm, int64_t ncell,
                                                    const int32_t* __restrict__ gate,
-                                                   const float* __restrict__ r, Grid g) {
-  cell_sort_body<DIM>(cell_start, unsorted, perm, iperm, ncell, gate, blockIdx.x, r, g);
+                                                   const float* __restrict__ r, Grid g,
+                                                   int32_t* __restrict__ clear) {
+  cell_sort_body<DIM>(cell_start, unsorted, perm, iperm, ncell, gate, blockIdx.x, r, g, clear);
 }
 
 template <int DIM>
@@ -846,40 +934,103 @@ __global__ void k_needs_rebuild(const float* __restrict__ r, const float* __rest
 
 // ----------------------------------------------------------- idx writer
 __global__ void k_counts_orig(const int32_t* __restrict__ perm, const int32_t* __restrict__ cnt,
-                              int64_t* __restrict__ cnt64, int n, int npad, int tpp) {
+                              int32_t* __restrict__ cnt_id, int n, int npad, int tpp) {
   int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= n) return;
-  int64_t c = 0;
+  int c = 0;
   for (int h = 0; h < tpp; ++h) c += cnt[h * npad + s];
-  cnt64[perm[s]] = c;
+  cnt_id[perm[s]] = c;
 }
 
-// Receivers of sender a in sub-list order (lane 0's list, then lane 1's, ...).
-__global__ void k_write_idx(const int32_t* __restrict__ perm, const int32_t* __restrict__ cnt,
-                            const int32_t* __restrict__ ell, const int64_t* __restrict__ off,
-                            int32_t* __restrict__ idx, int64_t max_occ, int n, int npad, int tpp,
-                            int lane_width) {
-  int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= n) return;
-  const int a = perm[s];
-  int64_t p = off[a];
-  for (int h = 0; h < tpp; ++h) {
-    const int c = cnt[h * npad + s];
-    const int32_t* lst = ell + ((int64_t)h * lane_width) * npad + s;
-    for (int k = 0; k < c && p < max_occ; ++k, ++p) {
-      idx[p] = perm[lst[(int64_t)k * npad]];
-      idx[max_occ + p] = a;
+// Receivers of each sender in sub-list order (sub-list 0, then 1, ...), written
+// to its segment off[sender] of idx.  A workgroup takes kIdxTile consecutive
+// sorted senders: it reads kIdxRows rows of every sub-list at a time (a row is
+// contiguous over the senders), looks the ids up, and turns the tile around
+// through LDS, so that a wavefront writes one sender's receivers side by side.
+// Ten rows are in flight a thread: waiting for each (ids and all) took 531 us
+// where this takes 488 us (1,000,000 particles, 113 pairs each: 1.35 GB at
+// 2.8 TB/s, bound by stores that start and end inside cache lines); a thread
+// per sender, which wrote 4 B here and there, took 4,824 us.
+constexpr int kIdxTile = 32, kIdxRows = 40;
+
+template <int TPP>
+__global__ __launch_bounds__(kBlock) void k_write_idx(
+    const int32_t* __restrict__ perm, const int32_t* __restrict__ cnt,
+    const int32_t* __restrict__ ell, const int64_t* __restrict__ off, int32_t* __restrict__ idx,
+    int64_t max_occ, int n, int npad, int lane_width) {
+  __shared__ int32_t tile[TPP][kIdxRows][kIdxTile + 1];
+  __shared__ int32_t own[kIdxTile];  // the sender
+  __shared__ int64_t seg[kIdxTile];  // its segment
+  __shared__ int32_t count[TPP][kIdxTile];
+  __shared__ int rows;  // the longest sub-list of the tile
+  const int s0 = blockIdx.x * kIdxTile;
+  const int ns = min(kIdxTile, n - s0);
+  if (threadIdx.x == 0) rows = 0;
+  __syncthreads();
+  if (threadIdx.x < kIdxTile) {
+    const int c = threadIdx.x;
+    own[c] = c < ns ? perm[s0 + c] : 0;
+    seg[c] = c < ns ? off[own[c]] : 0;
+    for (int h = 0; h < TPP; ++h) count[h][c] = c < ns ? cnt[h * npad + s0 + c] : 0;
+    atomicMax(&rows, count[0][c]);  // sub-list 0 is never shorter than the others
+  }
+  __syncthreads();
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  constexpr int kLoads = 10;  // rows a thread has in flight
+  static_assert(TPP * kIdxRows * kIdxTile % (kLoads * kBlock) == 0, "whole batches of loads");
+  for (int k0 = 0; k0 < rows; k0 += kIdxRows) {
+    for (int t0 = threadIdx.x; t0 < TPP * kIdxRows * kIdxTile; t0 += kLoads * kBlock) {
+      int32_t j[kLoads];
+#pragma unroll
+      for (int q = 0; q < kLoads; ++q) {
+        const int t = t0 + q * kBlock;
+        const int c = t % kIdxTile, k = k0 + t / kIdxTile % kIdxRows, h = t / (kIdxTile * kIdxRows);
+        j[q] = -1;
+        if (k < count[h][c]) j[q] = ell[((int64_t)h * lane_width + k) * npad + s0 + c];
+      }
+#pragma unroll
+      for (int q = 0; q < kLoads; ++q)
+        if (j[q] >= 0) j[q] = perm[j[q]];
+#pragma unroll
+      for (int q = 0; q < kLoads; ++q) {
+        const int t = t0 + q * kBlock;
+        tile[t / (kIdxTile * kIdxRows)][t / kIdxTile % kIdxRows][t % kIdxTile] = j[q];
+      }
     }
+    __syncthreads();
+    for (int c = wave; c < ns; c += kBlock / 64) {
+      const int a = own[c];
+      int64_t p0 = seg[c] + k0;
+#pragma unroll
+      for (int h = 0; h < TPP; ++h) {
+        const int m = count[h][c];
+        const int64_t p = p0 + lane;
+        if (lane < kIdxRows && k0 + lane < m && p < max_occ) {
+          idx[p] = tile[h][lane][c];
+          idx[max_occ + p] = a;
+        }
+        p0 += m;
+      }
+    }
+    __syncthreads();
   }
 }
 
-__global__ void k_pad_idx(int32_t* __restrict__ idx, int64_t max_occ,
-                          const int64_t* __restrict__ total, int n) {
-  int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p < max_occ && p >= *total) {
+// Entries *total .. max_occ of both rows hold n.
+constexpr int kPadBlocks = 2048;
+__global__ __launch_bounds__(kBlock) void k_pad_idx(int32_t* __restrict__ idx, int64_t max_occ,
+                                                    const int64_t* __restrict__ total, int n) {
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t p = *total + (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < max_occ;
+       p += stride) {
     idx[p] = n;
     idx[max_occ + p] = n;
   }
+}
+
+static unsigned pad_blocks(int64_t max_occ) {
+  const int64_t b = cdiv(max_occ, kBlock);
+  return (unsigned)(b < kPadBlocks ? b : kPadBlocks);
 }
 
 // idx of a skin list: the pairs of each sender (sub-list order) that pass the
@@ -888,7 +1039,7 @@ __global__ void k_pad_idx(int32_t* __restrict__ idx, int64_t max_occ,
 struct SkinIdxArgs {
   const float* r;
   const int32_t *perm, *cnt, *ell;
-  int64_t* cnt64;
+  int32_t* cnt_id;
   const int64_t* off;
   int32_t* idx;
   int64_t max_occ;
@@ -920,7 +1071,7 @@ __global__ void k_skin_pairs(SkinIdxArgs a) {
       ++p;
     }
   }
-  if (!WRITE) a.cnt64[i] = p;
+  if (!WRITE) a.cnt_id[i] = (int32_t)p;
 }
 
 __global__ void k_chunk_budget(const int64_t* __restrict__ off, int n, int64_t n_sub,
@@ -945,29 +1096,12 @@ Grid make_grid(const sph_nl_config& c) {
   return g;
 }
 
-// Bins r into `bank`: hash + histogram, scan, scatter, per-cell sort, positions.
-__global__ void k_bin_init(int64_t* __restrict__ info, const int64_t* __restrict__ prev,
-                           int32_t* __restrict__ count, int64_t ncell) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < ncell) count[i] = 0;
-  if (i == 0) {
-    info[0] = prev ? prev[0] : 0;
-    for (int k = 1; k < 8; ++k) info[k] = 0;
-  }
-}
-
-// Resets the error block and the cell histogram.
-int bin_init(sph_ws* ws, const int64_t* prev_info, int64_t* info, hipStream_t st) {
-  SPH_LAUNCH(ws, "bin_init", st,
-             k_bin_init<<<cdiv(ws->ncell, kBlock), kBlock, 0, st>>>(info, prev_info,
-                                                                   ws->cell_count, ws->ncell));
-  return SPH_OK;
-}
-
-// Kick/drift/wrap of the state fused with the histogram of the new positions.
+// Kick/drift/wrap of the state fused with the histogram of the new positions;
+// resets the error block.
 int integrate_and_hash(sph_ws* ws, const float* r, const float* u, const float* dudt,
                        const float* dvdt, float* r_out, float* u_out, float* v_out, float dt,
-                       float ctvf, const float* box, hipStream_t st) {
+                       float ctvf, const float* box, const int64_t* prev_info, int64_t* info,
+                       hipStream_t st) {
   const auto& c = ws->cfg;
   const int n = c.n;
   Grid g = make_grid(c);
@@ -975,12 +1109,12 @@ int integrate_and_hash(sph_ws* ws, const float* r, const float* u, const float* 
     SPH_LAUNCH(ws, "integrate_hash", st,
                k_integrate_hash<2><<<cdiv(n, kBlock), kBlock, 0, st>>>(
                    r, u, dudt, dvdt, r_out, u_out, v_out, n, dt, ctvf, g, box[0], box[1], 0.0f,
-                   ws->cell_count, ws->pcell, ws->pslot));
+                   ws->cell_count, ws->pcell, ws->pslot, info, prev_info));
   else
     SPH_LAUNCH(ws, "integrate_hash", st,
                k_integrate_hash<3><<<cdiv(n, kBlock), kBlock, 0, st>>>(
                    r, u, dudt, dvdt, r_out, u_out, v_out, n, dt, ctvf, g, box[0], box[1], box[2],
-                   ws->cell_count, ws->pcell, ws->pslot));
+                   ws->cell_count, ws->pcell, ws->pslot, info, prev_info));
   return SPH_OK;
 }
 
@@ -990,17 +1124,17 @@ int bin_finish(sph_ws* ws, int bank, const float* r, int64_t* info, hipStream_t 
   const auto& c = ws->cfg;
   const int n = c.n;
   Bank& B = ws->bank[bank];
-  SPH_LAUNCH(ws, "scan_cells", st,
-             (k_scan_single<int32_t, int32_t><<<1, kScanThreads, 0, st>>>(
-                 ws->cell_count, ws->ncell, B.cell_start, &info[2], info,
-                 c.use_cells ? (int64_t)c.cell_capacity : (int64_t)-1, ws->cell_count)));
+  const int rc = scan<int32_t>(ws, "scan_cells", ws->cell_count, ws->ncell, B.cell_start,
+                               (int32_t*)ws->scan_tmp, info,
+                               c.use_cells ? (int64_t)c.cell_capacity : (int64_t)-1, nullptr, st);
+  if (rc) return rc;
   SPH_LAUNCH(ws, "scatter", st,
              k_scatter<<<cdiv(n, kBlock), kBlock, 0, st>>>(ws->pcell, ws->pslot, B.cell_start,
                                                          ws->unsorted, n));
   SPH_LAUNCH(ws, "cell_sort", st,
              k_cell_sort<3><<<cdiv(ws->ncell * 64, 256), 256, 0, st>>>(
                  B.cell_start, ws->unsorted, B.perm, B.iperm, ws->ncell, nullptr, nullptr,
-                 Grid{}));
+                 Grid{}, ws->cell_count));
   if (!r) return SPH_OK;
   if (c.dim == 2)
     SPH_LAUNCH(ws, "gather_pos", st,
@@ -1016,16 +1150,14 @@ int bin_particles(sph_ws* ws, int bank, const float* r, const int64_t* prev_info
   const auto& c = ws->cfg;
   const int n = c.n;
   Grid g = make_grid(c);
-  int rc = bin_init(ws, prev_info, info, st);
-  if (rc) return rc;
   if (c.dim == 2)
     SPH_LAUNCH(ws, "hash_count", st,
-               k_hash_count<2><<<cdiv(n, kBlock), kBlock, 0, st>>>(r, n, g, ws->cell_count,
-                                                                 ws->pcell, ws->pslot, nullptr));
+               k_hash_count<2><<<cdiv(n, kBlock), kBlock, 0, st>>>(
+                   r, n, g, ws->cell_count, ws->pcell, ws->pslot, nullptr, info, prev_info));
   else
     SPH_LAUNCH(ws, "hash_count", st,
-               k_hash_count<3><<<cdiv(n, kBlock), kBlock, 0, st>>>(r, n, g, ws->cell_count,
-                                                                 ws->pcell, ws->pslot, nullptr));
+               k_hash_count<3><<<cdiv(n, kBlock), kBlock, 0, st>>>(
+                   r, n, g, ws->cell_count, ws->pcell, ws->pslot, nullptr, info, prev_info));
   return bin_finish(ws, bank, r, info, st);
 }
 
@@ -1141,21 +1273,22 @@ int skin_begin(sph_ws* ws, const float* r, const float* u, const float* dudt, co
     SPH_LAUNCH(ws, "skin_hash", st,
                k_hash_count<3><<<nb, kBlock, 0, st>>>(r_out, n, gs, S.cell_count, ws->pcell,
                                                       ws->pslot, S.flag));
-  SPH_LAUNCH(ws, "skin_scan", st,
-             (k_scan_single<int32_t, int32_t><<<1, kScanThreads, 0, st>>>(
-                 S.cell_count, S.ncell, S.b.cell_start, nullptr, nullptr, (int64_t)-1,
-                 S.cell_count, S.flag)));
+  const int rc = scan<int32_t>(ws, "skin_scan", S.cell_count, S.ncell, S.b.cell_start,
+                               (int32_t*)ws->scan_tmp, nullptr, -1, S.flag, st);
+  if (rc) return rc;
   SPH_LAUNCH(ws, "skin_scatter", st,
              k_scatter<<<nb, kBlock, 0, st>>>(ws->pcell, ws->pslot, S.b.cell_start, ws->unsorted,
                                               n, S.flag));
   if (c.dim == 2)
     SPH_LAUNCH(ws, "skin_sort", st,
                k_cell_sort<2><<<cdiv(S.ncell * 64, 256), 256, 0, st>>>(
-                   S.b.cell_start, ws->unsorted, S.b.perm, S.b.iperm, S.ncell, S.flag, r_out, gs));
+                   S.b.cell_start, ws->unsorted, S.b.perm, S.b.iperm, S.ncell, S.flag, r_out, gs,
+                   S.cell_count));
   else
     SPH_LAUNCH(ws, "skin_sort", st,
                k_cell_sort<3><<<cdiv(S.ncell * 64, 256), 256, 0, st>>>(
-                   S.b.cell_start, ws->unsorted, S.b.perm, S.b.iperm, S.ncell, S.flag, r_out, gs));
+                   S.b.cell_start, ws->unsorted, S.b.perm, S.b.iperm, S.ncell, S.flag, r_out, gs,
+                   S.cell_count));
   return SPH_OK;
 }
 
@@ -1226,12 +1359,10 @@ int pair_offsets(sph_ws* ws, int bank, hipStream_t st) {
   const int n = ws->cfg.n;
   Bank& B = ws->bank[bank];
   SPH_LAUNCH(ws, "counts_orig", st,
-             k_counts_orig<<<cdiv(n, kBlock), kBlock, 0, st>>>(B.perm, B.cnt, ws->cnt64, n,
+             k_counts_orig<<<cdiv(n, kBlock), kBlock, 0, st>>>(B.perm, B.cnt, ws->cnt_id, n,
                                                              ws->npad, ws->tpp));
-  SPH_LAUNCH(ws, "scan_pairs", st,
-             (k_scan_single<int64_t, int64_t><<<1, kScanThreads, 0, st>>>(
-                 ws->cnt64, n, ws->off64, nullptr, nullptr, -1)));
-  return SPH_OK;
+  return scan<int64_t>(ws, "scan_pairs", ws->cnt_id, n, ws->off64, ws->scan_tmp, nullptr, -1,
+                       nullptr, st);
 }
 
 // ------------------------------------------------------------ ensembles
@@ -1315,8 +1446,8 @@ __global__ void k_hash_count_ens(const EnsBin* __restrict__ t, const EnsBlock* _
 // one workgroup per member
 __global__ __launch_bounds__(kScanThreads) void k_scan_ens(const EnsBin* __restrict__ t) {
   const EnsBin& a = t[blockIdx.x];
-  scan_single_body<int32_t, int32_t>(a.cell_count, a.ncell, a.cell_start, nullptr, nullptr, -1,
-                                     a.cell_count, a.flag);
+  scan_body<int32_t>(a.cell_count, a.ncell, cdiv(a.ncell, kScanTile) * kScanTile, nullptr,
+                     a.cell_start, nullptr, -1, a.flag, 0, 1);
 }
 
 __global__ void k_scatter_ens(const EnsBin* __restrict__ t, const EnsBlock* __restrict__ map) {
@@ -1333,7 +1464,7 @@ __global__ __launch_bounds__(256) void k_cell_sort_ens(const EnsBin* __restrict_
   if (m.sim < 0) return;
   const EnsBin& a = t[m.sim];
   cell_sort_body<DIM>(a.cell_start, a.unsorted, a.perm, a.iperm, a.ncell, a.flag, m.blk, a.r,
-                      a.g);
+                      a.g, a.cell_count);
 }
 
 template <int DIM, int TPP>
@@ -1691,16 +1822,17 @@ extern "C" int sph_cell_list(int32_t dim, int32_t n, const float* r, const float
                                                                    pslot, nullptr));
   }
   // cell starts, the largest occupancy into info[2], CELL_LIST_OVERFLOW into info[0]
-  SPH_LAUNCH(ws, "scan_cells", st,
-             (k_scan_single<int32_t, int32_t><<<1, kScanThreads, 0, st>>>(
-                 counts, nc, start, &info[2], info, capacity)));
+  SPH_LAUNCH(ws, "fill", st, k_fill<int64_t><<<1, 64, 0, st>>>(info + 2, 1, 0));
+  const int rc = scan<int32_t>(ws, "scan_cells", counts, nc, start, nullptr, info, capacity,
+                               nullptr, st);
+  if (rc) return rc;
   if (n == 0) return SPH_OK;
   SPH_LAUNCH(ws, "scatter", st,
              k_scatter<<<cdiv(n, kBlock), kBlock, 0, st>>>(pcell, pslot, start, unsorted, n));
   // ascending id inside each cell: the order of the reference's stable argsort
   SPH_LAUNCH(ws, "cell_sort", st,
              k_cell_sort<3><<<cdiv(nc * 64, 256), 256, 0, st>>>(start, unsorted, perm, iperm, nc,
-                                                               nullptr, nullptr, Grid{}));
+                                                               nullptr, nullptr, Grid{}, nullptr));
   if (dim == 2)
     SPH_LAUNCH(ws, "cell_list_fill", st,
                k_cell_list_fill<2><<<cdiv(n, kBlock), kBlock, 0, st>>>(
@@ -1773,13 +1905,19 @@ extern "C" int sph_nl_write_idx(sph_ws* ws, int bank, int32_t* idx, int64_t max_
   if (rc) return rc;
   const int n = ws->cfg.n;
   Bank& B = ws->bank[bank];
-  SPH_LAUNCH(ws, "write_idx", st,
-             k_write_idx<<<cdiv(n, kBlock), kBlock, 0, st>>>(B.perm, B.cnt, B.ell, ws->off64, idx,
-                                                           max_occupancy, n, ws->npad, ws->tpp,
-                                                           ws->lane_width));
+  constexpr int T2 = tpp_of(2), T3 = tpp_of(3);
+  const dim3 grid((unsigned)cdiv(n, kIdxTile));
+  if (ws->cfg.dim == 2)
+    SPH_LAUNCH(ws, "write_idx", st,
+               (k_write_idx<T2><<<grid, kBlock, 0, st>>>(B.perm, B.cnt, B.ell, ws->off64, idx,
+                                                     max_occupancy, n, ws->npad, ws->lane_width)));
+  else
+    SPH_LAUNCH(ws, "write_idx", st,
+               (k_write_idx<T3><<<grid, kBlock, 0, st>>>(B.perm, B.cnt, B.ell, ws->off64, idx,
+                                                     max_occupancy, n, ws->npad, ws->lane_width)));
   SPH_LAUNCH(ws, "pad_idx", st,
-             k_pad_idx<<<cdiv(max_occupancy, kBlock), kBlock, 0, st>>>(idx, max_occupancy,
-                                                                      ws->off64 + n, n));
+             k_pad_idx<<<pad_blocks(max_occupancy), kBlock, 0, st>>>(idx, max_occupancy,
+                                                                    ws->off64 + n, n));
   (void)info;
   return SPH_OK;
 }
@@ -1802,7 +1940,7 @@ extern "C" int sph_nl_write_idx_skin(sph_ws* ws, const float* r, int32_t* idx,
   a.perm = ws->sk.b.perm;
   a.cnt = ws->sk.b.cnt;
   a.ell = ws->sk.b.ell;
-  a.cnt64 = ws->cnt64;
+  a.cnt_id = ws->cnt_id;
   a.off = ws->off64;
   a.idx = idx;
   a.max_occ = max_occupancy;
@@ -1820,15 +1958,15 @@ extern "C" int sph_nl_write_idx_skin(sph_ws* ws, const float* r, int32_t* idx,
     SPH_LAUNCH(ws, "skin_idx_count", st, (k_skin_pairs<2, false><<<nb, kBlock, 0, st>>>(a)));
   else
     SPH_LAUNCH(ws, "skin_idx_count", st, (k_skin_pairs<3, false><<<nb, kBlock, 0, st>>>(a)));
-  SPH_LAUNCH(ws, "scan_pairs", st,
-             (k_scan_single<int64_t, int64_t><<<1, kScanThreads, 0, st>>>(
-                 ws->cnt64, n, ws->off64, nullptr, nullptr, -1)));
+  const int rc = scan<int64_t>(ws, "scan_pairs", ws->cnt_id, n, ws->off64, ws->scan_tmp, nullptr,
+                               -1, nullptr, st);
+  if (rc) return rc;
   if (c.dim == 2)
     SPH_LAUNCH(ws, "skin_idx_write", st, (k_skin_pairs<2, true><<<nb, kBlock, 0, st>>>(a)));
   else
     SPH_LAUNCH(ws, "skin_idx_write", st, (k_skin_pairs<3, true><<<nb, kBlock, 0, st>>>(a)));
   SPH_LAUNCH(ws, "pad_idx", st,
-             k_pad_idx<<<cdiv(max_occupancy, kBlock), kBlock, 0, st>>>(idx, max_occupancy,
-                                                                      ws->off64 + n, n));
+             k_pad_idx<<<pad_blocks(max_occupancy), kBlock, 0, st>>>(idx, max_occupancy,
+                                                                    ws->off64 + n, n));
   return SPH_OK;
 }

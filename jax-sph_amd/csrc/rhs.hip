@@ -19,10 +19,10 @@
 namespace sph {
 
 // Bank helpers from nl.hip
-int bin_init(sph_ws* ws, const int64_t* prev_info, int64_t* info, hipStream_t st);
 int integrate_and_hash(sph_ws* ws, const float* r, const float* u, const float* dudt,
                        const float* dvdt, float* r_out, float* u_out, float* v_out, float dt,
-                       float ctvf, const float* box, hipStream_t st);
+                       float ctvf, const float* box, const int64_t* prev_info, int64_t* info,
+                       hipStream_t st);
 int bin_finish(sph_ws* ws, int bank, const float* r, int64_t* info, hipStream_t st);
 int build_pairs(sph_ws* ws, int bank, int64_t max_occupancy, int64_t* info, hipStream_t st);
 int skin_begin(sph_ws* ws, const float* r, const float* u, const float* dudt, const float* dvdt,
@@ -600,10 +600,8 @@ extern "C" int sph_step(sph_ws* ws, int bank, const sph_solver_params* prm, floa
     return skin_finish(ws, max_occupancy, info, st);
   }
   // 1. kick/drift into the output buffers, binned at the new positions
-  rc = bin_init(ws, prev_info, info, st);
-  if (rc) return rc;
   rc = integrate_and_hash(ws, in->r, in->u, in->dudt, in->dvdt, r_out, out->u, out->v, dt,
-                          tvf_coef, prm->box, st);
+                          tvf_coef, prm->box, prev_info, info, st);
   if (rc) return rc;
   rc = bin_finish(ws, bank, nullptr, info, st);
   if (rc) return rc;

@@ -64,8 +64,8 @@ struct sph_ws {
   int32_t* pslot = nullptr;       // N: arrival slot inside the cell
   int32_t* unsorted = nullptr;    // N: ids scattered by arrival order
   int64_t* off64 = nullptr;       // N + 1: pair offsets of the idx writer
-  int64_t* scan_tmp = nullptr;    // block carries of the scans
-  int64_t* cnt64 = nullptr;       // N: pair count per original id
+  int64_t* scan_tmp = nullptr;    // 1024: chunk sums of the scans
+  int32_t* cnt_id = nullptr;      // N: pair count per original id
   // per-workgroup (pairs, largest list) partials of the pair build and of the
   // counting density sweep, reduced by one workgroup (no same-address atomics)
   int64_t* part_build = nullptr;  // 2 * part_blocks
