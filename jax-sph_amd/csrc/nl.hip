@@ -16,6 +16,7 @@
 #include "ens.h"
 #include "sph_device.h"
 #include "sph_internal.h"
+#include "sweep.h"
 
 namespace sph {
 
@@ -222,20 +223,21 @@ __device__ __forceinline__ int integrate_block(
   return i;
 }
 
-// integrate_block fused with the cell hash and histogram of the new position.
-template <int DIM>
+// integrate_block fused with the cell hash and histogram of the new position
+// (HASH = false: the drift alone, for sets that k_bin_small bins).
+template <int DIM, bool HASH>
 __global__ __launch_bounds__(kBlock) void k_integrate_hash(
     const float* __restrict__ r, const float* __restrict__ u, const float* __restrict__ dudt,
     const float* __restrict__ dvdt, float* __restrict__ r_out, float* __restrict__ u_out,
     float* __restrict__ v_out, int n, float dt, float ctvf, Grid g, float bx, float by, float bz,
     int32_t* __restrict__ cell_count, int32_t* __restrict__ pcell, int32_t* __restrict__ pslot,
     int64_t* __restrict__ info, const int64_t* __restrict__ prev) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) reset_info(info, prev);
+  if (HASH && blockIdx.x == 0 && threadIdx.x == 0) reset_info(info, prev);
   const float side[3] = {bx, by, bz};
   float x[3] = {0.f, 0.f, 0.f};
   const int i = integrate_block<DIM>(r, u, dudt, dvdt, r_out, u_out, v_out, n, dt, ctvf, side,
                                      blockIdx.x, x);
-  if (i >= n) return;
+  if (!HASH || i >= n) return;
   int h = 0;
   if (g.use_cells) {
     int c[3];
@@ -284,13 +286,15 @@ __global__ void k_integrate_skin(const float* __restrict__ r, const float* __res
                                  float* __restrict__ v_out, int n, float dt, float ctvf, Grid g,
                                  float bx, float by, float bz, int32_t* __restrict__ cell_count,
                                  const float4* __restrict__ posb, float trigger_sq,
-                                 int32_t* __restrict__ flag) {
+                                 int32_t* __restrict__ flag, int64_t* __restrict__ info,
+                                 const int64_t* __restrict__ prev) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) reset_info(info, prev);
   integrate_skin_body<DIM>(r, u, dudt, dvdt, r_out, u_out, v_out, n, dt, ctvf, g, bx, by, bz,
                            cell_count, posb, trigger_sq, flag, blockIdx.x);
 }
 
-// Largest reference-grid cell occupancy of this step (one workgroup): sets
-// info[2] and the cell-capacity bit, resets the other info entries (keeping
+// Ensembles: largest reference-grid cell occupancy of this step (one workgroup
+// a member): sets info[2] and the cell-capacity bit, resets the other info entries (keeping
 // the sticky bits of prev[0]) and clears the histogram for the next step.
 constexpr int kCellsThreads = 1024;
 __device__ __forceinline__ void cells_max_body(int32_t* __restrict__ count, int64_t ncell,
@@ -320,14 +324,6 @@ __device__ __forceinline__ void cells_max_body(int32_t* __restrict__ count, int6
     for (int k = 1; k < 8; ++k) info[k] = 0;
     info[2] = mm;
   }
-}
-
-__global__ __launch_bounds__(kCellsThreads) void k_cells_max(int32_t* __restrict__ count,
-                                                             int64_t ncell,
-                                                             int64_t* __restrict__ info,
-                                                             const int64_t* __restrict__ prev,
-                                                             int64_t capacity) {
-  cells_max_body(count, ncell, info, prev, capacity);
 }
 
 __global__ void k_max_reduce(const int32_t* __restrict__ a, int64_t n, int64_t* __restrict__ out) {
@@ -609,6 +605,173 @@ __global__ __launch_bounds__(256) void k_cell_sort(const int32_t* __restrict__ c
   cell_sort_body<DIM>(cell_start, unsorted, perm, iperm, ncell, gate, blockIdx.x, r, g, clear);
 }
 
+// Hash and histogram of the skin grid, gated on the rebuild request; the first
+// cell_blocks workgroups instead take kCellsBlock cells each of this step's
+// reference-grid histogram: its largest entry into info[2] (reset by the drift)
+// with the cell-capacity bit, the histogram cleared for the next step.  They
+// ride in this launch because nothing in it depends on them.
+constexpr int kCellsBlock = 16 * kBlock;
+template <int DIM>
+__global__ __launch_bounds__(kBlock) void k_skin_hash(
+    const float* __restrict__ r, int n, Grid g, int32_t* __restrict__ cell_count,
+    int32_t* __restrict__ pcell, int32_t* __restrict__ pslot, const int32_t* __restrict__ flag,
+    int32_t* __restrict__ ref_count, int64_t ref_ncell, int cell_blocks,
+    int64_t* __restrict__ info, int64_t capacity) {
+  if ((int)blockIdx.x >= cell_blocks) {
+    hash_count_body<DIM>(r, n, g, cell_count, pcell, pslot, flag, blockIdx.x - cell_blocks);
+    return;
+  }
+  int m = 0;
+#pragma unroll
+  for (int q = 0; q < kCellsBlock / kBlock; ++q) {
+    const int64_t i = (int64_t)blockIdx.x * kCellsBlock + q * kBlock + threadIdx.x;
+    if (i < ref_ncell) {
+      m = max(m, ref_count[i]);
+      ref_count[i] = 0;
+    }
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_down(m, o, 64));
+  if ((threadIdx.x & 63) == 0 && m > 0) {
+    atomicMax((unsigned long long*)&info[2], (unsigned long long)m);
+    if (capacity >= 0 && m > capacity)
+      atomicOr((unsigned long long*)&info[0], (unsigned long long)SPH_CELL_LIST_OVERFLOW);
+  }
+}
+
+// Binning of a small particle set by one workgroup, with the histogram, the
+// ids and their sort keys in LDS: one launch instead of hash, scan, scatter and
+// sort, which a small set spends on launches (4 x 2-6 us).  The same cells and
+// the same order inside them.  SKIN: gated on the rebuild request, sub-cell
+// order, and before the gate the reference-grid occupancy as in k_skin_hash;
+// otherwise the error block is reset and receives the grid's own occupancy.
+// A thread takes kBinOwn particles and as many cells: up to kBinMax of each.
+// Microseconds a step by separate launches and so: skin step of 2,500 2D
+// particles 74.9 and 63.0, of 4,096 74.3 and 63.4, of 4,096 in 3D 90.5 and 88.8
+// (a rank among 38 particles a cell instead of 10); exact step 73.2 and 59.8,
+// 72.1 and 64.6, 141.6 and 142.1.  Larger sets have more than one workgroup
+// can do in the time of the launches saved.
+constexpr int kBinThreads = 1024;
+constexpr int kBinOwn = 4;
+constexpr int kBinMax = kBinOwn * kBinThreads;
+static bool bins_small(int n, int64_t ncell) { return n <= kBinMax && ncell <= kBinMax; }
+
+struct BinSmall {
+  const float* r;
+  int n;
+  Grid g;
+  int64_t ncell;
+  int32_t *cell_start, *perm, *iperm;
+  float4* pos;         // not SKIN, or null: the sorted positions
+  int32_t* ref_count;  // SKIN
+  int64_t ref_ncell;
+  int64_t* info;
+  const int64_t* prev;  // not SKIN
+  int64_t capacity;
+  const int32_t* gate;  // SKIN
+};
+
+template <int DIM, bool SKIN>
+__global__ __launch_bounds__(kBinThreads) void k_bin_small(BinSmall a) {
+  __shared__ int32_t start[kBinMax + 1];
+  __shared__ uint32_t keys[kBinMax];
+  __shared__ int32_t part[kBinThreads / 64];
+  __shared__ int32_t occ[kBinThreads / 64];
+  const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
+  int m = 0;
+  if (SKIN) {
+    for (int64_t i = t; i < a.ref_ncell; i += kBinThreads) {
+      m = max(m, a.ref_count[i]);
+      a.ref_count[i] = 0;
+    }
+  }
+  const bool run = !SKIN || *a.gate != 0;  // uniform
+  int cell[kBinOwn], slot[kBinOwn];
+  if (run) {
+#pragma unroll
+    for (int q = 0; q < kBinOwn; ++q) start[t + q * kBinThreads] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kBinOwn; ++q) {
+      const int i = t + q * kBinThreads;
+      cell[q] = slot[q] = 0;
+      if (i < a.n) {
+        if (a.g.use_cells) {
+          int c[3];
+          cell_coords<DIM>(load_pos<DIM>(a.r, i), a.g, c);
+          cell[q] = cell_hash<DIM>(c, a.g);
+        }
+        slot[q] = atomicAdd(&start[cell[q]], 1);
+      }
+    }
+    __syncthreads();
+    // exclusive scan: thread t takes cells 4t..4t+3
+    int v[kBinOwn], s = 0;
+#pragma unroll
+    for (int q = 0; q < kBinOwn; ++q) {
+      v[q] = start[kBinOwn * t + q];
+      s += v[q];
+      if (!SKIN) m = max(m, v[q]);
+    }
+    int inc = s;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(inc, o, 64);
+      if (lane >= o) inc += y;
+    }
+    if (lane == 63) part[wid] = inc;
+    __syncthreads();
+    int base = inc - s;
+#pragma unroll
+    for (int w = 0; w < kBinThreads / 64; ++w) base += w < wid ? part[w] : 0;
+#pragma unroll
+    for (int q = 0; q < kBinOwn; ++q) {
+      const int c = kBinOwn * t + q;
+      start[c] = base;
+      if (c <= a.ncell) a.cell_start[c] = base;
+      base += v[q];
+    }
+    if (t == kBinThreads - 1) {
+      start[kBinMax] = base;
+      if (a.ncell == kBinMax) a.cell_start[kBinMax] = base;
+    }
+    __syncthreads();
+    // sort keys: (sub-cell, id), ids below kBinMax
+    uint32_t key[kBinOwn];
+#pragma unroll
+    for (int q = 0; q < kBinOwn; ++q) {
+      const int i = t + q * kBinThreads;
+      if (i >= a.n) continue;
+      key[q] = (uint32_t)i;
+      if (SKIN) key[q] |= sub_cell_code<DIM>(load_pos<DIM>(a.r, i), a.g) * (uint32_t)kBinMax;
+      keys[start[cell[q]] + slot[q]] = key[q];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kBinOwn; ++q) {
+      const int i = t + q * kBinThreads;
+      if (i >= a.n) continue;
+      const int b = start[cell[q]], e = start[cell[q] + 1];
+      int rank = b;
+      for (int k = b; k < e; ++k) rank += keys[k] < key[q] ? 1 : 0;
+      a.perm[rank] = i;
+      a.iperm[i] = rank;
+      if (!SKIN && a.pos) a.pos[rank] = load_pos<DIM>(a.r, i);
+    }
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_down(m, o, 64));
+  if (lane == 0) occ[wid] = m;
+  __syncthreads();
+  if (t == 0) {
+    int mm = 0;
+    for (int w = 0; w < kBinThreads / 64; ++w) mm = max(mm, occ[w]);
+    if (!SKIN) reset_info(a.info, a.prev);
+    a.info[2] = mm;
+    if (a.capacity >= 0 && mm > a.capacity) a.info[0] |= SPH_CELL_LIST_OVERFLOW;
+  }
+}
+
 template <int DIM>
 __global__ void k_gather_pos(const float* __restrict__ r, const int32_t* __restrict__ perm,
                              float4* __restrict__ pos, int n) {
@@ -871,53 +1034,9 @@ __global__ void k_finalize(int64_t* __restrict__ info, int64_t max_occ) {
   if (threadIdx.x == 0 && info[1] > max_occ) info[0] |= SPH_NEIGHBOR_LIST_OVERFLOW;
 }
 
-// Reduces the per-workgroup (pairs, largest list) partials of one launch:
-// *tot_out = sum, *max_out = max (each nullable); with max_occ >= 0 also the
-// NEIGHBOR_LIST_OVERFLOW bit (partition.py:976).  With a gate, runs only when
-// *gate != 0; with clear_flag, zeroes *clear_flag at the end (the skin step's
-// rebuild request is consumed).
 constexpr int kReduceThreads = 1024;
-__device__ __forceinline__ void reduce_parts_body(const int64_t* __restrict__ part, int nblocks,
-                                                  int64_t* __restrict__ tot_out,
-                                                  int64_t* __restrict__ max_out,
-                                                  int64_t* __restrict__ info, int64_t max_occ,
-                                                  const int32_t* __restrict__ gate,
-                                                  int32_t* __restrict__ clear_flag) {
-  __shared__ int64_t ws_t[kReduceThreads / 64], ws_m[kReduceThreads / 64];
-  const bool run = !gate || *gate != 0;  // uniform
-  if (run) {
-    int64_t t = 0, m = 0;
-    for (int b = threadIdx.x; b < nblocks; b += kReduceThreads) {
-      t += part[2 * b];
-      m = part[2 * b + 1] > m ? part[2 * b + 1] : m;
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      t += __shfl_down(t, o, 64);
-      const int64_t y = __shfl_down(m, o, 64);
-      m = y > m ? y : m;
-    }
-    if ((threadIdx.x & 63) == 0) { ws_t[threadIdx.x >> 6] = t; ws_m[threadIdx.x >> 6] = m; }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      int64_t tt = 0, mm = 0;
-      for (int w = 0; w < kReduceThreads / 64; ++w) {
-        tt += ws_t[w];
-        mm = ws_m[w] > mm ? ws_m[w] : mm;
-      }
-      if (tot_out) *tot_out = tt;
-      if (max_out) *max_out = mm;
-      if (max_occ >= 0 && tt > max_occ) info[0] |= SPH_NEIGHBOR_LIST_OVERFLOW;
-    }
-  }
-  if (clear_flag && threadIdx.x == 0) *clear_flag = 0;
-}
-
-__global__ __launch_bounds__(kReduceThreads) void k_reduce_parts(
-    const int64_t* __restrict__ part, int nblocks, int64_t* __restrict__ tot_out,
-    int64_t* __restrict__ max_out, int64_t* __restrict__ info, int64_t max_occ,
-    const int32_t* __restrict__ gate, int32_t* __restrict__ clear_flag) {
-  reduce_parts_body(part, nblocks, tot_out, max_out, info, max_occ, gate, clear_flag);
+__global__ __launch_bounds__(kReduceThreads) void k_reduce_parts(Reduce a) {
+  reduce_parts_body<kReduceThreads>(a);
 }
 
 template <int DIM>
@@ -1105,25 +1224,35 @@ int integrate_and_hash(sph_ws* ws, const float* r, const float* u, const float* 
   const auto& c = ws->cfg;
   const int n = c.n;
   Grid g = make_grid(c);
-  if (c.dim == 2)
-    SPH_LAUNCH(ws, "integrate_hash", st,
-               k_integrate_hash<2><<<cdiv(n, kBlock), kBlock, 0, st>>>(
-                   r, u, dudt, dvdt, r_out, u_out, v_out, n, dt, ctvf, g, box[0], box[1], 0.0f,
-                   ws->cell_count, ws->pcell, ws->pslot, info, prev_info));
-  else
-    SPH_LAUNCH(ws, "integrate_hash", st,
-               k_integrate_hash<3><<<cdiv(n, kBlock), kBlock, 0, st>>>(
-                   r, u, dudt, dvdt, r_out, u_out, v_out, n, dt, ctvf, g, box[0], box[1], box[2],
-                   ws->cell_count, ws->pcell, ws->pslot, info, prev_info));
+  const auto kernel = bins_small(n, ws->ncell)
+                          ? (c.dim == 2 ? k_integrate_hash<2, false> : k_integrate_hash<3, false>)
+                          : (c.dim == 2 ? k_integrate_hash<2, true> : k_integrate_hash<3, true>);
+  SPH_LAUNCH(ws, "integrate_hash", st,
+             kernel<<<cdiv(n, kBlock), kBlock, 0, st>>>(
+                 r, u, dudt, dvdt, r_out, u_out, v_out, n, dt, ctvf, g, box[0], box[1],
+                 c.dim == 3 ? box[2] : 0.0f, ws->cell_count, ws->pcell, ws->pslot, info,
+                 prev_info));
   return SPH_OK;
 }
 
-// Scan of the histogram, scatter, per-cell id sort; then (if r is given) the
-// sorted positions the pair build reads.
-int bin_finish(sph_ws* ws, int bank, const float* r, int64_t* info, hipStream_t st) {
+// Order of the particles at r by cells and ids: scan of the histogram, scatter,
+// per-cell id sort (a small set in one launch, hash included); then (want_pos)
+// the sorted positions the pair build reads.
+int bin_finish(sph_ws* ws, int bank, const float* r, bool want_pos, const int64_t* prev_info,
+               int64_t* info, hipStream_t st) {
   const auto& c = ws->cfg;
   const int n = c.n;
   Bank& B = ws->bank[bank];
+  if (bins_small(n, ws->ncell)) {
+    const BinSmall b{r, n, make_grid(c), ws->ncell, B.cell_start, B.perm, B.iperm,
+                     want_pos ? B.pos : nullptr, nullptr, 0, info, prev_info,
+                     c.use_cells ? (int64_t)c.cell_capacity : (int64_t)-1, nullptr};
+    if (c.dim == 2)
+      SPH_LAUNCH(ws, "bin", st, (k_bin_small<2, false><<<1, kBinThreads, 0, st>>>(b)));
+    else
+      SPH_LAUNCH(ws, "bin", st, (k_bin_small<3, false><<<1, kBinThreads, 0, st>>>(b)));
+    return SPH_OK;
+  }
   const int rc = scan<int32_t>(ws, "scan_cells", ws->cell_count, ws->ncell, B.cell_start,
                                (int32_t*)ws->scan_tmp, info,
                                c.use_cells ? (int64_t)c.cell_capacity : (int64_t)-1, nullptr, st);
@@ -1135,7 +1264,7 @@ int bin_finish(sph_ws* ws, int bank, const float* r, int64_t* info, hipStream_t 
              k_cell_sort<3><<<cdiv(ws->ncell * 64, 256), 256, 0, st>>>(
                  B.cell_start, ws->unsorted, B.perm, B.iperm, ws->ncell, nullptr, nullptr,
                  Grid{}, ws->cell_count));
-  if (!r) return SPH_OK;
+  if (!want_pos) return SPH_OK;
   if (c.dim == 2)
     SPH_LAUNCH(ws, "gather_pos", st,
                k_gather_pos<2><<<cdiv(n, kBlock), kBlock, 0, st>>>(r, B.perm, B.pos, n));
@@ -1150,18 +1279,16 @@ int bin_particles(sph_ws* ws, int bank, const float* r, const int64_t* prev_info
   const auto& c = ws->cfg;
   const int n = c.n;
   Grid g = make_grid(c);
-  if (c.dim == 2)
+  if (!bins_small(n, ws->ncell)) {
+    const auto kernel = c.dim == 2 ? k_hash_count<2> : k_hash_count<3>;
     SPH_LAUNCH(ws, "hash_count", st,
-               k_hash_count<2><<<cdiv(n, kBlock), kBlock, 0, st>>>(
+               kernel<<<cdiv(n, kBlock), kBlock, 0, st>>>(
                    r, n, g, ws->cell_count, ws->pcell, ws->pslot, nullptr, info, prev_info));
-  else
-    SPH_LAUNCH(ws, "hash_count", st,
-               k_hash_count<3><<<cdiv(n, kBlock), kBlock, 0, st>>>(
-                   r, n, g, ws->cell_count, ws->pcell, ws->pslot, nullptr, info, prev_info));
-  return bin_finish(ws, bank, r, info, st);
+  }
+  return bin_finish(ws, bank, r, true, prev_info, info, st);
 }
 
-int build_pairs(sph_ws* ws, int bank, int64_t max_occupancy, int64_t* info, hipStream_t st) {
+int build_pairs(sph_ws* ws, int bank, int64_t* info, hipStream_t st) {
   const auto& c = ws->cfg;
   Bank& B = ws->bank[bank];
   BuildArgs a;
@@ -1208,12 +1335,14 @@ int build_pairs(sph_ws* ws, int bank, int64_t max_occupancy, int64_t* info, hipS
     else
       SPH_LAUNCH(ws, "nl_build", st, (k_nl_build<3, T3, false, true><<<grid, kBlock, 0, st>>>(a)));
   }
-  // occupancy info[1], largest list info[3], and the overflow bit when max_occupancy >= 0
-  SPH_LAUNCH(ws, "reduce_pairs", st,
-             k_reduce_parts<<<1, kReduceThreads, 0, st>>>(ws->part_build, (int)grid.x, &info[1],
-                                                          &info[3], info, max_occupancy,
-                                                          nullptr, nullptr));
   return SPH_OK;
+}
+
+// What an exact build leaves to reduce: occupancy info[1], largest list
+// info[3], and the overflow bit when max_occupancy >= 0.
+Reduce build_tail(sph_ws* ws, int64_t max_occupancy, int64_t* info) {
+  const int blocks = (int)xcd_grid(cdiv((int64_t)ws->cfg.n * ws->tpp, kBlock), ws->xcd_remap);
+  return Reduce{ws->part_build, blocks, &info[1], &info[3], info, max_occupancy, nullptr, nullptr};
 }
 
 // The exact-predicate band of the pair build: squared distances (fp32, minimum
@@ -1256,23 +1385,34 @@ int skin_begin(sph_ws* ws, const float* r, const float* u, const float* dudt, co
     SPH_LAUNCH(ws, "integrate_skin", st,
                k_integrate_skin<2><<<nb, kBlock, 0, st>>>(
                    r, u, dudt, dvdt, r_out, u_out, v_out, n, dt, ctvf, g, box[0], box[1], 0.0f,
-                   ws->cell_count, S.posb, S.trigger_sq, S.flag));
+                   ws->cell_count, S.posb, S.trigger_sq, S.flag, info, prev_info));
   else
     SPH_LAUNCH(ws, "integrate_skin", st,
                k_integrate_skin<3><<<nb, kBlock, 0, st>>>(
                    r, u, dudt, dvdt, r_out, u_out, v_out, n, dt, ctvf, g, box[0], box[1], box[2],
-                   ws->cell_count, S.posb, S.trigger_sq, S.flag));
-  SPH_LAUNCH(ws, "cells_max", st,
-             k_cells_max<<<1, kCellsThreads, 0, st>>>(ws->cell_count, ws->ncell, info, prev_info,
-                                                      (int64_t)c.cell_capacity));
+                   ws->cell_count, S.posb, S.trigger_sq, S.flag, info, prev_info));
+  if (bins_small(n, S.ncell)) {
+    const BinSmall b{r_out, n, gs, S.ncell, S.b.cell_start, S.b.perm, S.b.iperm, nullptr,
+                     ws->cell_count, ws->ncell, info, nullptr, (int64_t)c.cell_capacity, S.flag};
+    if (c.dim == 2)
+      SPH_LAUNCH(ws, "skin_bin", st, (k_bin_small<2, true><<<1, kBinThreads, 0, st>>>(b)));
+    else
+      SPH_LAUNCH(ws, "skin_bin", st, (k_bin_small<3, true><<<1, kBinThreads, 0, st>>>(b)));
+    return SPH_OK;
+  }
+  const int cb = (int)cdiv(ws->ncell, kCellsBlock);
   if (c.dim == 2)
     SPH_LAUNCH(ws, "skin_hash", st,
-               k_hash_count<2><<<nb, kBlock, 0, st>>>(r_out, n, gs, S.cell_count, ws->pcell,
-                                                      ws->pslot, S.flag));
+               k_skin_hash<2><<<nb + cb, kBlock, 0, st>>>(r_out, n, gs, S.cell_count, ws->pcell,
+                                                         ws->pslot, S.flag, ws->cell_count,
+                                                         ws->ncell, cb, info,
+                                                         (int64_t)c.cell_capacity));
   else
     SPH_LAUNCH(ws, "skin_hash", st,
-               k_hash_count<3><<<nb, kBlock, 0, st>>>(r_out, n, gs, S.cell_count, ws->pcell,
-                                                      ws->pslot, S.flag));
+               k_skin_hash<3><<<nb + cb, kBlock, 0, st>>>(r_out, n, gs, S.cell_count, ws->pcell,
+                                                         ws->pslot, S.flag, ws->cell_count,
+                                                         ws->ncell, cb, info,
+                                                         (int64_t)c.cell_capacity));
   const int rc = scan<int32_t>(ws, "skin_scan", S.cell_count, S.ncell, S.b.cell_start,
                                (int32_t*)ws->scan_tmp, nullptr, -1, S.flag, st);
   if (rc) return rc;
@@ -1336,22 +1476,22 @@ int skin_build(sph_ws* ws, int64_t* info, hipStream_t st) {
     SPH_LAUNCH(ws, "skin_build", st, (k_nl_build<2, T2, false, false><<<grid, kBlock, 0, st>>>(a)));
   else
     SPH_LAUNCH(ws, "skin_build", st, (k_nl_build<3, T3, false, false><<<grid, kBlock, 0, st>>>(a)));
-  // largest skin list of one particle -> info[7] (only on a rebuild)
-  SPH_LAUNCH(ws, "reduce_skin", st,
-             k_reduce_parts<<<1, kReduceThreads, 0, st>>>(ws->part_build, (int)grid.x, nullptr,
-                                                          &info[7], info, -1, S.flag, nullptr));
   return SPH_OK;
+}
+
+// What a skin build leaves to reduce: the largest list of one particle ->
+// info[7] (only on a rebuild).
+Reduce skin_build_tail(sph_ws* ws, int64_t* info) {
+  const int blocks = (int)xcd_grid(cdiv((int64_t)ws->cfg.n * ws->tpp, kBlock), ws->xcd_remap);
+  return Reduce{ws->part_build, blocks, nullptr, &info[7], info, -1, ws->sk.flag, nullptr};
 }
 
 // End of a skin-list step: occupancy and largest list from the counting
 // density sweep's partials, the overflow bit, and the rebuild request is consumed.
-int skin_finish(sph_ws* ws, int64_t max_occupancy, int64_t* info, hipStream_t st) {
-  const int64_t blocks = xcd_grid(cdiv((int64_t)ws->cfg.n * ws->tpp, kBlock), ws->xcd_remap);
-  SPH_LAUNCH(ws, "reduce_pairs", st,
-             k_reduce_parts<<<1, kReduceThreads, 0, st>>>(ws->part_sweep, (int)blocks, &info[1],
-                                                          &info[3], info, max_occupancy,
-                                                          nullptr, ws->sk.flag));
-  return SPH_OK;
+Reduce skin_step_tail(sph_ws* ws, int64_t max_occupancy, int64_t* info) {
+  const int blocks = (int)xcd_grid(cdiv((int64_t)ws->cfg.n * ws->tpp, kBlock), ws->xcd_remap);
+  return Reduce{ws->part_sweep, blocks, &info[1], &info[3], info, max_occupancy, nullptr,
+                ws->sk.flag};
 }
 
 // pair counts per original id and their exclusive scan (off64[0..N])
@@ -1399,23 +1539,14 @@ struct EnsBin {  // skin-grid binning, all gated on the member's rebuild flag
   int32_t *unsorted, *perm, *iperm;
 };
 
-struct EnsReduce {
-  const int64_t* part;
-  int nblocks;
-  int64_t *tot_out, *max_out, *info;
-  int64_t max_occ;
-  const int32_t* gate;
-  int32_t* clear_flag;
-};
-
 struct EnsNL {
   int n = 0;
   EnsInteg* integ = nullptr;
   EnsCells* cells = nullptr;
   EnsBin* bin = nullptr;
   BuildArgs* build = nullptr;
-  EnsReduce* red_build = nullptr;
-  EnsReduce* red_sweep = nullptr;
+  Reduce* red_build = nullptr;
+  Reduce* red_sweep = nullptr;
 };
 
 template <int DIM>
@@ -1477,10 +1608,8 @@ __global__ __launch_bounds__(kBlock, 6) void k_nl_build_ens(const BuildArgs* __r
 
 // one workgroup per member
 __global__ __launch_bounds__(kReduceThreads) void k_reduce_parts_ens(
-    const EnsReduce* __restrict__ t) {
-  const EnsReduce& a = t[blockIdx.x];
-  reduce_parts_body(a.part, a.nblocks, a.tot_out, a.max_out, a.info, a.max_occ, a.gate,
-                    a.clear_flag);
+    const Reduce* __restrict__ t) {
+  reduce_parts_body<kReduceThreads>(t[blockIdx.x]);
 }
 
 template <typename T>
@@ -1498,7 +1627,7 @@ int ens_nl_create(const std::vector<EnsMember>& members, EnsNL** out) {
   std::vector<EnsCells> cells(n);
   std::vector<EnsBin> bin(n);
   std::vector<BuildArgs> build(n);
-  std::vector<EnsReduce> rb(n), rs(n);
+  std::vector<Reduce> rb(n), rs(n);
   for (int k = 0; k < n; ++k) {
     const EnsMember& m = members[k];
     sph_ws* ws = m.ws;
@@ -1513,9 +1642,9 @@ int ens_nl_create(const std::vector<EnsMember>& members, EnsNL** out) {
     bin[k] = EnsBin{m.r_out, c.n, skin_grid(ws), S.cell_count, ws->pcell, ws->pslot, S.flag,
                     S.b.cell_start, S.ncell, ws->unsorted, S.b.perm, S.b.iperm};
     build[k] = skin_build_args(ws, m.info);
-    rb[k] = EnsReduce{ws->part_build, (int)lane_blocks, nullptr, &m.info[7], m.info, -1, S.flag,
+    rb[k] = Reduce{ws->part_build, (int)lane_blocks, nullptr, &m.info[7], m.info, -1, S.flag,
                       nullptr};
-    rs[k] = EnsReduce{ws->part_sweep, (int)lane_blocks, &m.info[1], &m.info[3], m.info,
+    rs[k] = Reduce{ws->part_sweep, (int)lane_blocks, &m.info[1], &m.info[3], m.info,
                       m.max_occupancy, nullptr, S.flag};
   }
   EnsNL* t = new EnsNL;
@@ -1872,7 +2001,11 @@ extern "C" int sph_nl_build(sph_ws* ws, int bank, const float* r, const int64_t*
   if (!r || !info) { set_error("sph_nl_build: null"); return SPH_ERR_ARG; }
   rc = bin_particles(ws, bank, r, prev_info, info, st);
   if (rc) return rc;
-  return build_pairs(ws, bank, max_occupancy, info, st);
+  rc = build_pairs(ws, bank, info, st);
+  if (rc) return rc;
+  SPH_LAUNCH(ws, "reduce_pairs", st,
+             k_reduce_parts<<<1, kReduceThreads, 0, st>>>(build_tail(ws, max_occupancy, info)));
+  return SPH_OK;
 }
 
 extern "C" int sph_nl_finalize(sph_ws* ws, int64_t max_occupancy, int64_t* info, hipStream_t st) {

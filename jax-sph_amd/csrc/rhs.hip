@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cmath>
+#include <cstring>
 #include <string>
 
 #include "ens.h"
@@ -23,13 +24,16 @@ int integrate_and_hash(sph_ws* ws, const float* r, const float* u, const float* 
                        const float* dvdt, float* r_out, float* u_out, float* v_out, float dt,
                        float ctvf, const float* box, const int64_t* prev_info, int64_t* info,
                        hipStream_t st);
-int bin_finish(sph_ws* ws, int bank, const float* r, int64_t* info, hipStream_t st);
-int build_pairs(sph_ws* ws, int bank, int64_t max_occupancy, int64_t* info, hipStream_t st);
+int bin_finish(sph_ws* ws, int bank, const float* r, bool want_pos, const int64_t* prev_info,
+               int64_t* info, hipStream_t st);
+int build_pairs(sph_ws* ws, int bank, int64_t* info, hipStream_t st);
+Reduce build_tail(sph_ws* ws, int64_t max_occupancy, int64_t* info);
+Reduce skin_build_tail(sph_ws* ws, int64_t* info);
+Reduce skin_step_tail(sph_ws* ws, int64_t max_occupancy, int64_t* info);
 int skin_begin(sph_ws* ws, const float* r, const float* u, const float* dudt, const float* dvdt,
                float* r_out, float* u_out, float* v_out, float dt, float ctvf, const float* box,
                const int64_t* prev_info, int64_t* info, hipStream_t st);
 int skin_build(sph_ws* ws, int64_t* info, hipStream_t st);
-int skin_finish(sph_ws* ws, int64_t max_occupancy, int64_t* info, hipStream_t st);
 
 // ------------------------------------------------------------- delta-SPH
 // Renormalisation matrix of solver.py:42-58: M = sum_j (-r_ij) (x) grad W_ij V_j
@@ -521,13 +525,18 @@ int ens_sweeps(EnsRHS* t, int dim, const SweepPlan& plan, const EnsMap& lanes, s
 
 namespace {
 
-// The sweeps of one list (density ... force), one launch each.
+// The sweeps of one list (density ... force), one launch each; on_density and
+// on_force (part null: nothing) ride in those launches.
 template <int DIM>
-int launch_kind(sph_ws* ws, SweepArgs& a, hipStream_t st) {
+int launch_kind(sph_ws* ws, SweepArgs& a, const Reduce& on_density, const Reduce& on_force,
+                hipStream_t st) {
   const SweepPlan pl = plan_of(a.prm);
   select_records(a, pl);
-  const dim3 grid(xcd_grid(cdivl((int64_t)a.n * tpp_of(DIM), kB), a.remap));
+  const unsigned blocks = xcd_grid(cdivl((int64_t)a.n * tpp_of(DIM), kB), a.remap);
   return for_plan_kind<DIM>(pl, [&](const char* name, SweepKernel k, EnsSweepKernel) -> int {
+    const bool density = !std::strcmp(name, "density"), force = !std::strcmp(name, "force");
+    a.tail = density ? on_density : force ? on_force : Reduce{};
+    const unsigned grid = blocks + (a.tail.part ? 1 : 0);
     SPH_LAUNCH(ws, name, st, (k<<<grid, kB, 0, st>>>(a)));
     return 0;
   });
@@ -547,12 +556,12 @@ extern "C" int sph_forward(sph_ws* ws, int bank, const sph_solver_params* prm,
     SPH_LAUNCH(ws, "gather_state", st,
                k_gather_state<2><<<grid, kB, 0, st>>>(a, in->r, in->u, in->v, nullptr, nullptr,
                                                       nullptr));
-    return launch_kind<2>(ws, a, st);
+    return launch_kind<2>(ws, a, Reduce{}, Reduce{}, st);
   }
   SPH_LAUNCH(ws, "gather_state", st,
              k_gather_state<3><<<grid, kB, 0, st>>>(a, in->r, in->u, in->v, nullptr, nullptr,
                                                     nullptr));
-  return launch_kind<3>(ws, a, st);
+  return launch_kind<3>(ws, a, Reduce{}, Reduce{}, st);
 }
 
 extern "C" int sph_step(sph_ws* ws, int bank, const sph_solver_params* prm, float dt, float tvf_coef,
@@ -595,15 +604,15 @@ extern "C" int sph_step(sph_ws* ws, int bank, const sph_solver_params* prm, floa
     a.in.u = out->u;
     a.in.v = out->v;
     a.info = info;
-    rc = dim == 2 ? launch_kind<2>(ws, a, st) : launch_kind<3>(ws, a, st);
-    if (rc) return rc;
-    return skin_finish(ws, max_occupancy, info, st);
+    const Reduce built = skin_build_tail(ws, info), done = skin_step_tail(ws, max_occupancy, info);
+    return dim == 2 ? launch_kind<2>(ws, a, built, done, st)
+                    : launch_kind<3>(ws, a, built, done, st);
   }
   // 1. kick/drift into the output buffers, binned at the new positions
   rc = integrate_and_hash(ws, in->r, in->u, in->dudt, in->dvdt, r_out, out->u, out->v, dt,
                           tvf_coef, prm->box, prev_info, info, st);
   if (rc) return rc;
-  rc = bin_finish(ws, bank, nullptr, info, st);
+  rc = bin_finish(ws, bank, r_out, false, prev_info, info, st);
   if (rc) return rc;
   // 2. sorted records (also the positions of the pair build), then the pairs
   SweepArgs a = make_args(ws, bank, prm, in, out);
@@ -618,13 +627,15 @@ extern "C" int sph_step(sph_ws* ws, int bank, const sph_solver_params* prm, floa
     SPH_LAUNCH(ws, "gather_state", st,
                k_gather_state<3><<<grid, kB, 0, st>>>(a, r_out, out->u, out->v, nl_pos, nullptr,
                                                       nullptr));
-  rc = build_pairs(ws, bank, max_occupancy, info, st);
+  rc = build_pairs(ws, bank, info, st);
   if (rc) return rc;
   // 3. forward + case hook
   a.in.r = r_out;
   a.in.u = out->u;
   a.in.v = out->v;
-  return dim == 2 ? launch_kind<2>(ws, a, st) : launch_kind<3>(ws, a, st);
+  const Reduce built = build_tail(ws, max_occupancy, info);
+  return dim == 2 ? launch_kind<2>(ws, a, built, Reduce{}, st)
+                  : launch_kind<3>(ws, a, built, Reduce{}, st);
 }
 
 extern "C" int sph_kernel_eval(int32_t kind, int32_t dim, float one_over_h, float sigma,

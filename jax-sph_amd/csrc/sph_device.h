@@ -269,11 +269,13 @@ __device__ __forceinline__ Eos make_eos(const sph_solver_params& p) {
 // [x * per, (x + 1) * per): cell-sorted particles that share neighbours then
 // share one L2 instead of being spread over all eight.
 constexpr int kXcds = 8;
-__device__ __forceinline__ int logical_block(int remap) {
-  const int b = blockIdx.x;
+__device__ __forceinline__ int logical_block_of(int b, int blocks, int remap) {
   if (!remap) return b;
-  const int per = gridDim.x / kXcds;
+  const int per = blocks / kXcds;
   return (b % kXcds) * per + b / kXcds;
+}
+__device__ __forceinline__ int logical_block(int remap) {
+  return logical_block_of(blockIdx.x, gridDim.x, remap);
 }
 __host__ __device__ inline unsigned xcd_grid(long long blocks, int remap) {
   return (unsigned)(remap ? (blocks + kXcds - 1) / kXcds * kXcds : blocks);

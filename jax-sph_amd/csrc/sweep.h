@@ -113,6 +113,52 @@ struct Recs {
   float4 *W1, *W2, *W3;                // (v - u, p) after density, walls, renormalisation
 };
 
+// Reduces the per-workgroup (pairs, largest list) partials of an earlier
+// launch: *tot_out = sum, *max_out = max (each nullable); with max_occ >= 0
+// also the NEIGHBOR_LIST_OVERFLOW bit (partition.py:976).  With a gate, runs
+// only when *gate != 0; with clear_flag, zeroes *clear_flag at the end (the
+// skin step's rebuild request is consumed).
+struct Reduce {
+  const int64_t* part;
+  int nblocks;
+  int64_t *tot_out, *max_out, *info;
+  int64_t max_occ;
+  const int32_t* gate;
+  int32_t* clear_flag;
+};
+
+template <int THREADS>
+__device__ __forceinline__ void reduce_parts_body(const Reduce& a) {
+  __shared__ int64_t ws_t[THREADS / 64], ws_m[THREADS / 64];
+  const bool run = !a.gate || *a.gate != 0;  // uniform
+  if (run) {
+    int64_t t = 0, m = 0;
+    for (int b = threadIdx.x; b < a.nblocks; b += THREADS) {
+      t += a.part[2 * b];
+      m = a.part[2 * b + 1] > m ? a.part[2 * b + 1] : m;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      t += __shfl_down(t, o, 64);
+      const int64_t y = __shfl_down(m, o, 64);
+      m = y > m ? y : m;
+    }
+    if ((threadIdx.x & 63) == 0) { ws_t[threadIdx.x >> 6] = t; ws_m[threadIdx.x >> 6] = m; }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      int64_t tt = 0, mm = 0;
+      for (int w = 0; w < THREADS / 64; ++w) {
+        tt += ws_t[w];
+        mm = ws_m[w] > mm ? ws_m[w] : mm;
+      }
+      if (a.tot_out) *a.tot_out = tt;
+      if (a.max_out) *a.max_out = mm;
+      if (a.max_occ >= 0 && tt > a.max_occ) a.info[0] |= SPH_NEIGHBOR_LIST_OVERFLOW;
+    }
+  }
+  if (a.clear_flag && threadIdx.x == 0) *a.clear_flag = 0;
+}
+
 struct SweepArgs {
   sph_solver_params prm;
   sph_state_in in;
@@ -139,6 +185,10 @@ struct SweepArgs {
   int64_t* info;  // non-null: the density sweep counts pairs (per-workgroup partials in part)
   int64_t* part;  // [2 * gridDim.x] pairs and largest list of each workgroup
   int remap;      // XCD-contiguous block order (grid a multiple of 8)
+  // tail.part non-null: the launch has one workgroup more, its first, which
+  // reduces the partials of an earlier launch (a launch of its own costs the
+  // stream 4-5 us, and nothing of this sweep reads the result)
+  Reduce tail;
 };
 
 // Pair (sweep centre s, listed j) of the neighbour set: the reference predicate
@@ -264,7 +314,13 @@ __global__ void k_gather_state(SweepArgs a, const float* __restrict__ r, const f
 #define SPH_SWEEP_KERNELS(NAME, RUN, TPARAMS, TARGS, MINW)                                \
   template <SPH_UNPAREN TPARAMS>                                                          \
   __global__ __launch_bounds__(kB, MINW) void NAME(SweepArgs a) {                         \
-    RUN<SPH_UNPAREN TARGS>(a, logical_block(a.remap));                                    \
+    const int extra = a.tail.part != nullptr;                                             \
+    if (extra && blockIdx.x == 0) {                                                       \
+      reduce_parts_body<kB>(a.tail);                                                      \
+      return;                                                                             \
+    }                                                                                     \
+    RUN<SPH_UNPAREN TARGS>(a, logical_block_of(blockIdx.x - extra, gridDim.x - extra,     \
+                                               a.remap));                                 \
   }                                                                                       \
   template <SPH_UNPAREN TPARAMS>                                                          \
   __global__ __launch_bounds__(kB, MINW) void NAME##_ens(const SweepArgs* __restrict__ t, \
@@ -653,6 +709,7 @@ inline SweepArgs make_args(sph_ws* ws, int bank, const sph_solver_params* prm, c
   }
   a.info = nullptr;
   a.part = ws->part_sweep;
+  a.tail = Reduce{};
   a.remap = ws->xcd_remap;
   a.Uf = a.R.U1; a.Vf = a.R.V0; a.Qf = a.R.Q1;
   a.Ud = a.R.U1; a.Qd = a.R.Q1;
