@@ -12,6 +12,7 @@
 #include <cmath>
 #include <mutex>
 #include <string>
+#include <type_traits>
 
 #include "ens.h"
 #include "sph_device.h"
@@ -794,8 +795,15 @@ struct BuildArgs {
   // fast filter: squared distances of the cell-adjacent image below `lo` are
   // in, above `hi` out; the band [lo, hi) bounds the difference between that
   // and the exact reference metric, and is decided by the exact predicate.
+  // (Skin lists: lo = hi, no band.  A skin list must hold every pair within
+  // cutoff + 0.98 skin, the most two particles can close before the next
+  // rebuild, so rounding at its outer edge cannot drop a pair that matters.)
   float lo, hi;
   int fast;
+  // the matrix-core filter of k_nl_tile: below tlo in, at or above thi out,
+  // in between the filter above decides
+  float tlo, thi;
+  int range;  // consecutive sorted particles whose pieces a workgroup of k_nl_tile takes
   int n, npad, lane_width, mask_self;
   int64_t* part;          // [2 * gridDim.x]: pairs found and largest list, per workgroup
   int64_t trunc_bits;     // error bits raised when a sub-list overflows
@@ -820,11 +828,7 @@ struct BuildArgs {
 // build's registers allow.
 constexpr int kStage = 24;
 
-// BAND = false (skin lists): pairs are kept by the fast squared distance
-// alone.  A skin list must hold every pair within cutoff + 0.98 skin (the
-// most two particles can close before the next rebuild), so rounding at its
-// outer edge, cutoff + skin, cannot drop a pair that matters.
-template <int DIM, int TPP, bool ORDERED, bool BAND>
+template <int DIM, int TPP, bool ORDERED>
 __device__ __forceinline__ void test_range(const BuildArgs& a, int s, int h, const float4 ps,
                                            int sid, int lo, int hi, const float* img,
                                            int32_t* __restrict__ out0, int32_t* stage0,
@@ -840,31 +844,15 @@ __device__ __forceinline__ void test_range(const BuildArgs& a, int s, int h, con
     unsigned mask = 0u;
     for (int t0 = 0; t0 < nb; t0 += G) {
       float4 pg[G];
-      if (BAND) {
 #pragma unroll
-        for (int u = 0; u < G; ++u) {
-          const int b = c0 + (t0 + u) * TPP;
-          const int bc = b < hi ? b : hi - 1;
-          __builtin_assume(bc >= 0);  // sorted slots: no sign extension in the address
-          pg[u] = a.pos[bc];
-        }
-      } else {
-        // skin builds read past the range into the padded tail (kSkinPosPad),
-        // from one address with constant offsets; those candidates are masked
-        // off below
-        __builtin_assume(c0 >= 0);
-        const float4* __restrict__ pb = a.pos + (c0 + t0 * TPP);
-#pragma unroll
-        for (int u = 0; u < G; ++u) pg[u] = pb[u * TPP];
+      for (int u = 0; u < G; ++u) {
+        const int b = c0 + (t0 + u) * TPP;
+        const int bc = b < hi ? b : hi - 1;
+        __builtin_assume(bc >= 0);  // sorted slots: no sign extension in the address
+        pg[u] = a.pos[bc];
       }
       unsigned got = 0u;  // bit u: candidate t0 + u is a pair
-      if (!BAND) {
-#pragma unroll
-        for (int u = 0; u < G; ++u) {
-          const float4 pb = pg[u];
-          got |= dist2<DIM>(sx - pb.x, sy - pb.y, sz - pb.z) < a.lo ? 1u << u : 0u;
-        }
-      } else if (a.fast) {
+      if (a.fast) {
         bool near = false;  // some candidate lies in the band around the cutoff
 #pragma unroll
         for (int u = 0; u < G; ++u) {
@@ -930,12 +918,49 @@ __device__ __forceinline__ void test_range(const BuildArgs& a, int s, int h, con
   }
 }
 
+// Per-workgroup partials of a build: total pairs (sum of the threads' shares)
+// and the largest list.  Every thread of the workgroup calls it.
+__device__ __forceinline__ void build_partials(int64_t* __restrict__ part, int blk, int share,
+                                               int count) {
+  __shared__ unsigned long long tot[kBlock / 64];
+  __shared__ int mx[kBlock / 64];
+  unsigned long long v = (unsigned long long)share;
+  int m = count;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    v += __shfl_down(v, o, 64);
+    int y = __shfl_down(m, o, 64);
+    m = y > m ? y : m;
+  }
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  if (lane == 0) { tot[wid] = v; mx[wid] = m; }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    unsigned long long t = 0;
+    int mm = 0;
+    for (int w = 0; w < kBlock / 64; ++w) { t += tot[w]; mm = mx[w] > mm ? mx[w] : mm; }
+    part[2 * blk] = (int64_t)t;
+    part[2 * blk + 1] = mm;
+  }
+}
+
+// The counts of a particle's sub-list h of `share` hits (of `count`), and the
+// overflow report of a particle whose sub-lists were truncated.
+template <int TPP, typename Args>
+__device__ __forceinline__ void store_count(const Args& a, int s, int h, int share, int count) {
+  a.cnt[h * a.npad + s] = share < a.lane_width ? share : a.lane_width;
+  if (h == 0 && count > TPP * a.lane_width) {  // some sub-list of s was truncated
+    atomicAdd((unsigned long long*)&a.info[5], 1ull);
+    if (a.trunc_bits) atomicOr((unsigned long long*)&a.info[0], (unsigned long long)a.trunc_bits);
+  }
+}
+
 // TPP lanes per sorted particle (the sender): each visits the 3^d cells around
 // the particle's own cell as 3^(d-1) contiguous x-strips, keeps its share of
 // the receivers with d^2 < cutoff^2 and stores them in its own sub-list.
 // blk: the workgroup's block within this list's grid; it also indexes the
 // workgroup's partials.
-template <int DIM, int TPP, bool ORDERED, bool BAND>
+template <int DIM, int TPP, bool ORDERED>
 __device__ __forceinline__ void nl_build_body(const BuildArgs& a, const int blk) {
   __shared__ int32_t stage_buf[kStage][kBlock];
   if (a.gate && *a.gate == 0) return;  // uniform over the list's grid
@@ -949,7 +974,7 @@ __device__ __forceinline__ void nl_build_body(const BuildArgs& a, const int blk)
     int32_t* stage = &stage_buf[0][threadIdx.x - h];    // stage column of lane 0 of s
     float img[3] = {0.0f, 0.0f, 0.0f};
     if (!a.g.use_cells) {
-      test_range<DIM, TPP, ORDERED, BAND>(a, s, h, ps, sid, 0, a.n, img, out, stage, count);
+      test_range<DIM, TPP, ORDERED>(a, s, h, ps, sid, 0, a.n, img, out, stage, count);
     } else {
       int c[3];
       cell_coords<DIM>(ps, a.g, c);
@@ -969,16 +994,16 @@ __device__ __forceinline__ void nl_build_body(const BuildArgs& a, const int blk)
           const int row = (cz * ny + cy) * nx;
           if (c[0] >= 1 && c[0] + 1 < nx) {
             img[0] = 0.0f;
-            test_range<DIM, TPP, ORDERED, BAND>(a, s, h, ps, sid, a.cell_start[row + c[0] - 1],
-                                          a.cell_start[row + c[0] + 2], img, out, stage, count);
+            test_range<DIM, TPP, ORDERED>(a, s, h, ps, sid, a.cell_start[row + c[0] - 1],
+                                    a.cell_start[row + c[0] + 2], img, out, stage, count);
           } else {
             for (int dx = -1; dx <= 1; ++dx) {
               int cx = c[0] + dx;
               img[0] = 0.0f;
               if (cx < 0) { cx += nx; img[0] = -a.box[0]; }
               else if (cx >= nx) { cx -= nx; img[0] = a.box[0]; }
-              test_range<DIM, TPP, ORDERED, BAND>(a, s, h, ps, sid, a.cell_start[row + cx],
-                                            a.cell_start[row + cx + 1], img, out, stage, count);
+              test_range<DIM, TPP, ORDERED>(a, s, h, ps, sid, a.cell_start[row + cx],
+                                      a.cell_start[row + cx + 1], img, out, stage, count);
             }
           }
         }
@@ -995,39 +1020,354 @@ __device__ __forceinline__ void nl_build_body(const BuildArgs& a, const int blk)
     int staged = share < kStage ? share : kStage;
     staged = staged < a.lane_width ? staged : a.lane_width;  // never past the sub-list
     for (int k = 0; k < staged; ++k) out[(int64_t)k * a.npad] = stage[k * kBlock];
-    a.cnt[h * a.npad + s] = share < a.lane_width ? share : a.lane_width;
-    if (h == 0 && count > TPP * a.lane_width) {  // some sub-list of s was truncated
-      atomicAdd((unsigned long long*)&a.info[5], 1ull);
-      if (a.trunc_bits) atomicOr((unsigned long long*)&a.info[0], (unsigned long long)a.trunc_bits);
-    }
+    store_count<TPP>(a, s, h, share, count);
   }
-  // block reductions: total pairs (sum of the lanes' shares) and the largest
-  // per-particle count
-  __shared__ unsigned long long tot[kBlock / 64];
-  __shared__ int mx[kBlock / 64];
-  unsigned long long v = (unsigned long long)share;
-  int m = count;
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    v += __shfl_down(v, o, 64);
-    int y = __shfl_down(m, o, 64);
-    m = y > m ? y : m;
-  }
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  if (lane == 0) { tot[wid] = v; mx[wid] = m; }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    unsigned long long t = 0;
-    int mm = 0;
-    for (int w = 0; w < kBlock / 64; ++w) { t += tot[w]; mm = mx[w] > mm ? mx[w] : mm; }
-    a.part[2 * blk] = (int64_t)t;
-    a.part[2 * blk + 1] = mm;
-  }
+  build_partials(a.part, blk, share, count);
 }
 
-template <int DIM, int TPP, bool ORDERED, bool BAND>
+template <int DIM, int TPP, bool ORDERED>
 __global__ __launch_bounds__(kBlock, ORDERED ? 1 : 6) void k_nl_build(BuildArgs a) {
-  nl_build_body<DIM, TPP, ORDERED, BAND>(a, logical_block(a.remap));
+  nl_build_body<DIM, TPP, ORDERED>(a, logical_block(a.remap));
+}
+
+// ------------------------------------------------- pair build, matrix cores
+// The same lists as nl_build_body (hits in candidate order, dealt round-robin),
+// for the unordered builds of a grid whose cell-adjacent image decides.  A
+// wavefront takes up to tile_rows particles of one cell (a "piece").  Their
+// candidates, the 3^(d-1) strips of cells (3^d cells at a face), are numbered
+// one after another and taken 64 at a time, one a lane; v_mfma_f32_4x4x1 with
+// the particles' block broadcast then gives 4 particles x 64 candidates of
+//   |a|^2 + |b|^2 - 2 a.b,   a, b relative to the cell's centre,
+// one particle a register, one candidate a lane, so a comparison's lane mask is
+// that particle's hits in candidate order: a hit's number is a count of the
+// mask's lower bits, and only the store to the stage runs for hits alone.
+// Squares within a band of the cutoff are decided by the filter of
+// nl_build_body.
+// Bound by the issue of instructions (vector 61%, scalar 64% of the cycles), 10
+// for a particle and 64 candidates; a lane that tests candidates of its own
+// takes 9 per candidate and 25 per hit, in a loop as long as the wavefront's
+// longest.  Exact list of 1,000,000 3D particles 647 -> 421 us; tiled() has the
+// other sizes.
+// A stage entry is 16 bits (segment and offset in it, from which the sorted
+// index follows), so that 7 workgroups' stages fit a CU's LDS; entries past
+// the stage, and those of segments over 2,047 long, go straight to the buffer.
+constexpr int kTileSegBits = 11;
+constexpr int kCandBits = 27;  // the same in a register: 5 bits of segment, 27 of offset
+static_assert(kCandBits - kTileSegBits == 16, "an entry is the halves of a code, or'ed");
+constexpr int tile_stage(int dim) { return dim == 3 ? 176 : 48; }
+// Particles of a piece: a 3D cell's 28 to 38 in two or three, a 2D cell's 9 to
+// 11 in one (with 16 rows, seven of them idle, 150 us at 810,000 particles).
+constexpr int tile_rows(int dim) { return dim == 3 ? 16 : 12; }
+
+__device__ __forceinline__ int lane_i(int x, int l) { return __builtin_amdgcn_readlane(x, l); }
+__device__ __forceinline__ float lane_f(float x, int l) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l));
+}
+
+template <int Q, int NQ, typename F>
+__device__ __forceinline__ void for_blocks(F&& f) {
+  f(std::integral_constant<int, Q>{});
+  if constexpr (Q + 1 < NQ) for_blocks<Q + 1, NQ>(f);
+}
+
+// The arguments stay in memory (read by scalar loads, again for each piece and
+// in the rare paths): all of them beside a count for each particle are more
+// than the scalar registers hold, and a spilled one costs vector instructions.
+using ColdArgs = const __attribute__((address_space(4))) BuildArgs;
+__device__ __forceinline__ ColdArgs* again(ColdArgs* a) {
+  asm volatile("" : "+s"(a));
+  return a;
+}
+
+// R: consecutive sorted particles of a workgroup, which takes the pieces that
+// start there (tile_range, or what the caller's grid makes of it).
+template <int DIM, int TPP>
+__device__ __forceinline__ void nl_tile_body(ColdArgs* args, const int blk, const int R) {
+  constexpr int W = kBlock / 64, S = tile_stage(DIM), P = tile_rows(DIM);
+  constexpr int kRowLanes = 16;        // lane l: particle l mod 16 of the piece
+  constexpr int L = 64 / kRowLanes;    // and one of so many for it in the write-out
+  static_assert(P <= kRowLanes, "a lane a particle");
+  typedef float v4f __attribute__((ext_vector_type(4)));
+  typedef unsigned long long mask_t;
+  using Entry = __attribute__((address_space(3))) uint16_t;
+  // rows of an odd number of words: the lanes that read one entry of each
+  // particle fall on different banks
+  constexpr int kRow = S + 2;
+  static_assert(kRow / 2 % 2 == 1, "odd row length");
+  __shared__ uint16_t stage_buf[W][P * kRow];
+  const int32_t* gate = args->gate;
+  if (gate && *gate == 0) return;  // uniform over the list's grid
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n = args->n;
+  const float4* __restrict__ pos = args->pos;
+  const uint16_t* stage = stage_buf[wv];
+  // entry 0 of row 0, counted in entries from the start of the LDS
+  const unsigned row0 = (unsigned)(uintptr_t)(Entry*)stage / 2;
+  const int p = lane % kRowLanes, part = lane / kRowLanes;
+  int found = 0, most_found = 0;  // pairs and largest list of this wavefront's pieces
+  const int end = min(n, (blk + 1) * R);
+  for (int g0 = blk * R; g0 < end; g0 += 64) {
+    // ---- the cells of 64 particles, one a lane, the same in every wavefront
+    const int s = g0 + lane < end ? g0 + lane : end - 1;
+    int cc[3] = {0, 0, 0}, cell_lo, cell_hi;
+    {
+      const Grid g = {{args->g.cs[0], args->g.cs[1], args->g.cs[2]},
+                      {args->g.cps[0], args->g.cps[1], args->g.cps[2]}, 1};
+      cell_coords<DIM>(pos[s], g, cc);
+      const int32_t* start = args->cell_start + cell_hash<DIM>(cc, g);
+      cell_lo = start[0];
+      cell_hi = start[1];
+    }
+    // the particles that start a piece; the wavefronts take them in turn
+    mask_t pieces = __ballot(g0 + lane < end && (unsigned)(s - cell_lo) % P == 0u);
+    for (int turn = 0; pieces; ++turn) {
+      const int l = __ffsll((long long)pieces) - 1;
+      pieces &= pieces - 1ull;
+      if (turn % W != wv) continue;
+      ColdArgs* const a = again(args);
+      const int s0 = g0 + l;
+      const int np = min(P, lane_i(cell_hi, l) - s0);
+      const int nx = a->g.cps[0], ny = a->g.cps[1], nz = DIM == 3 ? a->g.cps[2] : 1;
+      const int cx = lane_i(cc[0], l), cy = lane_i(cc[1], l);
+      const int cz = DIM == 3 ? lane_i(cc[2], l) : 0;
+      const float4 ps = pos[s0 + (p < np ? p : np - 1)];
+      // ---- its segments of candidates, one a lane, in the order of the cells
+      const bool face = cx < 1 || cx + 1 >= nx;
+      const int nseg = (DIM == 3 ? 9 : 3) * (face ? 3 : 1);
+      int lo = 0, len = 0;
+      float ix = 0.0f, iy = 0.0f, iz = 0.0f;  // image of the segment's cells
+      if (lane < nseg) {
+        const int strip = face ? lane / 3 : lane;
+        int x = face ? cx + lane % 3 - 1 : cx - 1;
+        int y = cy + strip % 3 - 1, z = DIM == 3 ? cz + strip / 3 - 1 : 0;
+        if (x < 0) { x += nx; ix = -a->box[0]; }
+        else if (x >= nx) { x -= nx; ix = a->box[0]; }
+        if (y < 0) { y += ny; iy = -a->box[1]; }
+        else if (y >= ny) { y -= ny; iy = a->box[1]; }
+        if (z < 0) { z += nz; iz = -a->box[2]; }
+        else if (z >= nz) { z -= nz; iz = a->box[2]; }
+        const int32_t* start = a->cell_start + (z * ny + y) * nx + x;
+        lo = start[0];
+        len = start[face ? 1 : 3] - lo;
+      }
+      const bool image = __ballot(ix != 0.0f || iy != 0.0f || iz != 0.0f) != 0ull;
+      // entries a particle can stage
+      const int room = __ballot(len >= 1 << kTileSegBits) != 0ull ? 0 : S;
+      // inclusive scan over 32 lanes, a row of 16 at a time
+      int pre = len;
+      pre += __builtin_amdgcn_update_dpp(0, pre, 0x111, 0xf, 0xf, true);  // row_shr:1
+      pre += __builtin_amdgcn_update_dpp(0, pre, 0x112, 0xf, 0xf, true);
+      pre += __builtin_amdgcn_update_dpp(0, pre, 0x114, 0xf, 0xf, true);
+      pre += __builtin_amdgcn_update_dpp(0, pre, 0x118, 0xf, 0xf, true);
+      int total = lane_i(pre, 15);
+      pre += lane >= 16 ? total : 0;
+      total = lane_i(pre, 31);
+      pre -= len;
+      const int shift = lo - pre;                     // sorted index of a candidate
+      const unsigned code = ((unsigned)lane << kCandBits) - (unsigned)pre;  // and its code
+      // particle s0's number as a candidate (in the middle segment), for mask_self
+      const int self0 = a->mask_self ? s0 - lane_i(shift, nseg / 2) : -(1 << 30);
+      // ---- the particles, relative to the cell's centre
+      const float csx = a->g.cs[0], csy = a->g.cs[1], csz = a->g.cs[2];
+      const float ox = ((float)cx + 0.5f) * csx, oy = ((float)cy + 0.5f) * csy;
+      const float oz = DIM == 3 ? ((float)cz + 0.5f) * csz : 0.0f;
+      float ax = ps.x - ox, ay = ps.y - oy, az = DIM == 3 ? ps.z - oz : 0.0f;
+      float aa = dist2<DIM>(ax, ay, az);
+      // d below is the square less `mid`; hits are under -width, and the
+      // exact filter decides within width
+      const float mid = 0.5f * (a->tlo + a->thi);
+      float width = 0.5f * (a->thi - a->tlo);
+      const bool inside = fabsf(ax) <= csx && fabsf(ay) <= csy && (DIM == 2 || fabsf(az) <= csz);
+      ax *= -2.0f;
+      ay *= -2.0f;
+      az *= -2.0f;
+      if (__ballot(!inside)) {
+        // a particle outside its cell (unwrapped positions are clamped into
+        // the grid) or not finite: the filter's bounds do not hold, and every
+        // candidate of the piece is left to the exact one
+        aa = ax = ay = az = 0.0f;
+        width = INFINITY;
+      }
+      if (p >= np) aa = INFINITY;  // no particle: no hits
+      int seg = 0;  // the last segment that starts before the candidates seen end
+      const int full = (int)row0 + room;
+      int tops = (int)row0;  // lane q: the next entry of row q, less q kRow
+      // Candidates are requested kDepth chunks before their tests (past the end:
+      // s0 again): a chunk's tests take less than a load that misses the L2.
+      constexpr int kDepth = 1;
+      unsigned codes[kDepth + 1];  // candidate c0 + 64 k + lane: segment and offset in it
+      // and its position, three words of it: a fourth that nothing reads would
+      // be some other value's register next, which then waits for the load
+      struct Xyz { float x, y, z; };
+      Xyz at[kDepth + 1];
+#pragma unroll
+      for (int k = 0; k <= kDepth; ++k) {
+        codes[k] = 0;
+        at[k] = Xyz{0.f, 0.f, 0.f};
+      }
+      for (int c0 = -64 * kDepth; c0 < total; c0 += 64) {
+        const int first_new = c0 + 64 * kDepth;
+        const int o = first_new + lane;
+        int to_j = lane_i(shift, seg);
+        unsigned to_c = (unsigned)lane_i((int)code, seg);
+        while (seg + 1 < nseg) {
+          const int first = lane_i(pre, seg + 1);
+          if (first >= first_new + 64) break;
+          ++seg;
+          const bool on = o >= first;
+          const int tj = lane_i(shift, seg), tc = lane_i((int)code, seg);
+          to_j = on ? tj : to_j;
+          to_c = on ? (unsigned)tc : to_c;
+        }
+        at[kDepth] = *(const Xyz*)(pos + (unsigned)(o < total ? o + to_j : s0));
+        codes[kDepth] = (unsigned)o + to_c;
+        const unsigned c = codes[0];
+        const float4 pb = make_float4(at[0].x, at[0].y, at[0].z, 0.0f);
+        if (c0 >= 0) {
+          const bool valid = c0 + lane < total;
+          float cix = 0.0f, ciy = 0.0f, ciz = 0.0f;  // its image
+          if (image) {
+            cix = __shfl(ix, (int)(c >> kCandBits), 64);
+            ciy = __shfl(iy, (int)(c >> kCandBits), 64);
+            if (DIM == 3) ciz = __shfl(iz, (int)(c >> kCandBits), 64);
+          }
+          const float bx = pb.x - (ox - cix), by = pb.y - (oy - ciy);
+          const float bz = DIM == 3 ? pb.z - (oz - ciz) : 0.0f;
+          const uint16_t entry = (uint16_t)((c >> (kCandBits - kTileSegBits)) | c);
+          const float bb = valid ? dist2<DIM>(bx, by, bz) - mid : INFINITY;
+          const v4f b4 = {bb, bb, bb, bb};
+          v4f d[P / 4];  // one chain a block, side by side
+          for_blocks<0, P / 4>([&](auto qc) {
+            constexpr int Q = decltype(qc)::value;
+            d[Q] = __builtin_amdgcn_mfma_f32_4x4x1f32(aa, 1.0f, b4, 4, Q, 0);
+          });
+          for_blocks<0, P / 4>([&](auto qc) {
+            constexpr int Q = decltype(qc)::value;
+            d[Q] = __builtin_amdgcn_mfma_f32_4x4x1f32(ax, bx, d[Q], 4, Q, 0);
+          });
+          for_blocks<0, P / 4>([&](auto qc) {
+            constexpr int Q = decltype(qc)::value;
+            d[Q] = __builtin_amdgcn_mfma_f32_4x4x1f32(ay, by, d[Q], 4, Q, 0);
+          });
+          if (DIM == 3)
+            for_blocks<0, P / 4>([&](auto qc) {
+              constexpr int Q = decltype(qc)::value;
+              d[Q] = __builtin_amdgcn_mfma_f32_4x4x1f32(az, bz, d[Q], 4, Q, 0);
+            });
+          const int self = c0 + lane - self0;  // the particle this candidate is, if any
+          if (__ballot(self >= 0 && self < np)) {
+#pragma unroll
+            for (int q = 0; q < P; ++q) d[q / 4][q % 4] = self == q ? INFINITY : d[q / 4][q % 4];
+          }
+          float nearest = INFINITY;
+#pragma unroll
+          for (int q = 0; q < P; ++q) nearest = fminf(nearest, fabsf(d[q / 4][q % 4]));
+          mask_t m[P];
+          int hits = 0;  // lane q: those of particle q
+#pragma unroll
+          for (int q = 0; q < P; ++q) {
+            m[q] = __ballot(d[q / 4][q % 4] < -width);
+            // one lane of hits (the compiler has no builtin for it)
+            asm("v_writelane_b32 %0, %1, %2" : "+v"(hits) : "s"((int)__popcll(m[q])), "n"(q));
+          }
+          if (__builtin_expect(__ballot(nearest < width || tops + hits > full) == 0ull, 1)) {
+            for_blocks<0, P / 4>([&](auto qc) {
+              constexpr int q0 = 4 * decltype(qc)::value;
+              if (q0 >= np) return;  // uniform
+#pragma unroll
+              for (int q = q0; q < q0 + 4; ++q) {
+                const unsigned k =
+                    __builtin_amdgcn_mbcnt_hi((unsigned)(m[q] >> 32),
+                                              __builtin_amdgcn_mbcnt_lo((unsigned)m[q], 0u));
+                const unsigned row = (unsigned)lane_i(tops, q);
+                Entry* const to = (Entry*)(uintptr_t)((k + row) << 1) + q * kRow;
+                if (__builtin_expect(__builtin_amdgcn_inverse_ballot_w64(m[q]), 1)) *to = entry;
+              }
+            });
+            tops += hits;
+          } else {
+            // the exact filter, particle by particle; hits past the stage go
+            // straight to the buffer
+            ColdArgs* const e = again(args);
+            const float box[3] = {e->box[0], e->box[1], e->box[2]};
+            const float half[3] = {e->half[0], e->half[1], e->half[2]};
+            const float flo = e->lo, fhi = e->hi, csq = e->cutoff_sq;
+            const int lane_width = e->lane_width;
+            const int cj =
+                __shfl(lo, (int)(c >> kCandBits), 64) + (int)(c & ((1u << kCandBits) - 1u));
+#pragma unroll 1
+            for (int q = 0; q < np; ++q) {
+              const float4 pq = make_float4(lane_f(ps.x, q), lane_f(ps.y, q),
+                                            DIM == 3 ? lane_f(ps.z, q) : 0.0f, 0.0f);
+              const float d2 = dist2<DIM>(pq.x - cix - pb.x, pq.y - ciy - pb.y,
+                                          DIM == 3 ? pq.z - ciz - pb.z : 0.0f);
+              const bool hit =
+                  valid && self != q &&
+                  (d2 < flo || (d2 < fhi && metric_sq_exact<DIM>(pq, pb, box, half) < csq));
+              const mask_t mq = __ballot(hit);
+              const int t = lane_i(tops, q);
+              const int k = t - (int)row0 +  // its number among the particle's hits
+                            (int)__builtin_amdgcn_mbcnt_hi(
+                                (unsigned)(mq >> 32),
+                                __builtin_amdgcn_mbcnt_lo((unsigned)mq, 0u));
+              if (hit && k < room)
+                *(Entry*)(uintptr_t)((k + row0 + q * kRow) << 1) = entry;
+              else if (hit && k / TPP < lane_width)
+                e->ell[((int64_t)(k % TPP) * lane_width + k / TPP) * e->npad + s0 + q] = cj;
+              tops = lane == q ? t + (int)__popcll(mq) : tops;
+            }
+          }
+        }
+#pragma unroll
+        for (int k = 0; k < kDepth; ++k) {
+          codes[k] = codes[k + 1];
+          at[k] = at[k + 1];
+        }
+      }
+      // ---- counts, and the staged entries in the order of the buffer's rows
+      const int own = __shfl(tops, p, 64) - (int)row0;  // 0 where there is no particle
+      int most = own;
+#pragma unroll
+      for (int o = kRowLanes / 2; o > 0; o >>= 1) most = max(most, __shfl_xor(most, o, 64));
+      most = __builtin_amdgcn_readfirstlane(most);
+      __builtin_amdgcn_wave_barrier();
+      ColdArgs* const b = again(args);
+      const int lane_width = b->lane_width, npad = b->npad;
+      found += part == 0 ? own : 0;
+      most_found = most > most_found ? most : most_found;
+      if (p < np && part < TPP)
+        store_count<TPP>(*b, s0 + p, part, (own + TPP - 1 - part) / TPP, own);
+      // hit k goes to sub-list k mod TPP at k / TPP
+      const int staged = min(p < np ? min(own, room) : 0, TPP * lane_width);
+      most = min(most, room);
+      int32_t* out = b->ell + ((int64_t)(part % TPP) * lane_width + part / TPP) * npad + s0 + p;
+      const int64_t row = (L / TPP) * (int64_t)npad;
+      constexpr int kAhead = 4;  // rows whose LDS reads are in flight together
+      for (int k0 = 0; k0 < most; k0 += L * kAhead) {
+        int e[kAhead], j[kAhead];
+#pragma unroll
+        for (int t = 0; t < kAhead; ++t)  // in the stage also past its last entry
+          e[t] = stage[min(min(p, P - 1) * kRow + k0 + L * t + part, P * kRow - 1)];
+#pragma unroll
+        for (int t = 0; t < kAhead; ++t)
+          j[t] = __shfl(lo, e[t] >> kTileSegBits, 64) + (e[t] & ((1 << kTileSegBits) - 1));
+#pragma unroll
+        for (int t = 0; t < kAhead; ++t) {
+          if (k0 + L * t + part < staged) *out = j[t];
+          out += row;
+        }
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+  }
+  build_partials(again(args)->part, blk, found, most_found);
+}
+
+template <int DIM, int TPP>
+__global__ __launch_bounds__(kBlock, 6) void k_nl_tile(BuildArgs) {
+  // the kernel's one argument, where it lies
+  ColdArgs* const args = (ColdArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+  nl_tile_body<DIM, TPP>(args, logical_block(args->remap), args->range);
 }
 
 __global__ void k_finalize(int64_t* __restrict__ info, int64_t max_occ) {
@@ -1288,6 +1628,56 @@ int bin_particles(sph_ws* ws, int bank, const float* r, const int64_t* prev_info
   return bin_finish(ws, bank, r, true, prev_info, info, st);
 }
 
+// The band of k_nl_tile's filter around cutoff_sq: outside it the filter of
+// nl_build_body decides the same.  Per component the exact metric is within
+// 2 ulp(box) of the true one, the fast square within 1 and this one (its
+// centre less an image) within 1: 2 reach sqrt(3) 3 ulp(box) < 16 reach
+// ulp(box).  The expanded square loses at most 15 2^-24 (|a| + |b|)^2, with
+// |a| + |b| <= sqrt(d) cell + reach for a pair at `reach`.
+static void tile_band(BuildArgs& a, float reach, int dim) {
+  double maxbox = 0.0, cell = 0.0;
+  for (int d = 0; d < dim; ++d) {
+    maxbox = std::fmax(maxbox, (double)a.box[d]);
+    cell = std::fmax(cell, (double)a.g.cs[d]);
+  }
+  const double ulp_box = std::nextafter((float)maxbox, INFINITY) - (float)maxbox;
+  const double m = std::sqrt((double)dim) * cell + reach;
+  const double band = 16.0 * reach * ulp_box + 16.0 * std::ldexp(m * m, -23);
+  a.tlo = (float)(a.cutoff_sq - band);
+  a.thi = (float)(a.cutoff_sq + band);
+}
+
+// The cell-adjacent image is the minimum image of every pair within the cutoff
+// when each side has >= 5 cells (2 cells < box/2).  Both the fast and the exact
+// squared distance are then within a few ulp(box) per component of the true
+// one (see cut_band).
+static bool fast_filter(const sph_nl_config& c) {
+  if (!c.use_cells) return false;
+  for (int d = 0; d < c.dim; ++d)
+    if (c.cps[d] < 5) return false;
+  return true;
+}
+
+// Which lists k_nl_tile builds: its filter is the fast one's, and ordered (half)
+// lists compare ids candidate by candidate.  In 2D its 64 candidates at a time
+// are two chunks half full for each 9 particles, which pays while SIMDs are
+// idle anyway; microseconds by k_nl_build and so (exact lists):
+//   2D 900 particles 25.2, 9.6; 10,000 24.4, 12.3; 40,000 26.0, 14.1;
+//   160,000 33.3, 33.9; 810,000 90, 130
+//   3D 8,000 84.9, 30.8; 64,000 97.1, 55.4; 262,144 221.6, 127.9;
+//   1,000,000 647, 421; Wendland C2 (18 a cell) 91,125 72.0, 36.1
+static bool tiled(const sph_nl_config& c) {
+  return fast_filter(c) && !c.ordered && (c.dim == 3 || c.n < 150000);
+}
+static bool skin_tiled(const sph_nl_config& c) { return c.dim == 3 || c.n < 150000; }
+
+static unsigned build_grid(const sph_ws* ws, bool tile) {
+  const auto& c = ws->cfg;
+  const int64_t blocks = tile ? cdiv(c.n, tile_range(c.dim, c.n))
+                              : cdiv((int64_t)c.n * ws->tpp, kBlock);
+  return xcd_grid(blocks, ws->xcd_remap);
+}
+
 int build_pairs(sph_ws* ws, int bank, int64_t* info, hipStream_t st) {
   const auto& c = ws->cfg;
   Bank& B = ws->bank[bank];
@@ -1314,34 +1704,23 @@ int build_pairs(sph_ws* ws, int bank, int64_t* info, hipStream_t st) {
   a.trunc_bits = ws->ell_overflow ? SPH_NEIGHBOR_LIST_OVERFLOW : 0;
   a.gate = nullptr;
   a.remap = ws->xcd_remap;
-  // The cell-adjacent image is the minimum image of every pair within the
-  // cutoff when each side has >= 5 cells (2 cells < box/2).  Both the fast and
-  // the exact squared distance are then within a few ulp(box) per component of
-  // the true one (see cut_band).
-  a.fast = c.use_cells ? 1 : 0;
-  for (int d = 0; d < c.dim; ++d)
-    if (c.cps[d] < 5) a.fast = 0;
+  a.fast = fast_filter(c);
+  a.range = tile_range(c.dim, c.n);
   cut_band(c, &a.lo, &a.hi);
+  tile_band(a, c.cutoff, c.dim);
   constexpr int T2 = tpp_of(2), T3 = tpp_of(3);
-  const dim3 grid(xcd_grid(cdiv((int64_t)c.n * (c.dim == 2 ? T2 : T3), kBlock), a.remap));
-  if (c.dim == 2) {
-    if (c.ordered)
-      SPH_LAUNCH(ws, "nl_build", st, (k_nl_build<2, T2, true, true><<<grid, kBlock, 0, st>>>(a)));
-    else
-      SPH_LAUNCH(ws, "nl_build", st, (k_nl_build<2, T2, false, true><<<grid, kBlock, 0, st>>>(a)));
-  } else {
-    if (c.ordered)
-      SPH_LAUNCH(ws, "nl_build", st, (k_nl_build<3, T3, true, true><<<grid, kBlock, 0, st>>>(a)));
-    else
-      SPH_LAUNCH(ws, "nl_build", st, (k_nl_build<3, T3, false, true><<<grid, kBlock, 0, st>>>(a)));
-  }
+  const bool d2 = c.dim == 2;
+  const auto kernel = tiled(c)    ? (d2 ? k_nl_tile<2, T2> : k_nl_tile<3, T3>)
+                      : c.ordered ? (d2 ? k_nl_build<2, T2, true> : k_nl_build<3, T3, true>)
+                                  : (d2 ? k_nl_build<2, T2, false> : k_nl_build<3, T3, false>);
+  SPH_LAUNCH(ws, "nl_build", st, (kernel<<<build_grid(ws, tiled(c)), kBlock, 0, st>>>(a)));
   return SPH_OK;
 }
 
 // What an exact build leaves to reduce: occupancy info[1], largest list
 // info[3], and the overflow bit when max_occupancy >= 0.
 Reduce build_tail(sph_ws* ws, int64_t max_occupancy, int64_t* info) {
-  const int blocks = (int)xcd_grid(cdiv((int64_t)ws->cfg.n * ws->tpp, kBlock), ws->xcd_remap);
+  const int blocks = (int)build_grid(ws, tiled(ws->cfg));
   return Reduce{ws->part_build, blocks, &info[1], &info[3], info, max_occupancy, nullptr, nullptr};
 }
 
@@ -1454,7 +1833,9 @@ static BuildArgs skin_build_args(sph_ws* ws, int64_t* info) {
   }
   a.cutoff_sq = S.reach_sq;
   a.fast = 1;
+  a.range = tile_range(c.dim, c.n);
   a.lo = a.hi = S.reach_sq;
+  tile_band(a, c.cutoff + S.skin, c.dim);
   a.n = c.n;
   a.npad = ws->npad;
   a.lane_width = S.lane_width;
@@ -1471,18 +1852,18 @@ int skin_build(sph_ws* ws, int64_t* info, hipStream_t st) {
   auto& S = ws->sk;
   const BuildArgs a = skin_build_args(ws, info);
   constexpr int T2 = tpp_of(2), T3 = tpp_of(3);
-  const dim3 grid(xcd_grid(cdiv((int64_t)c.n * (c.dim == 2 ? T2 : T3), kBlock), a.remap));
-  if (c.dim == 2)
-    SPH_LAUNCH(ws, "skin_build", st, (k_nl_build<2, T2, false, false><<<grid, kBlock, 0, st>>>(a)));
-  else
-    SPH_LAUNCH(ws, "skin_build", st, (k_nl_build<3, T3, false, false><<<grid, kBlock, 0, st>>>(a)));
+  const bool tile = skin_tiled(c);
+  const auto kernel = c.dim == 3 ? k_nl_tile<3, T3>
+                      : tile     ? k_nl_tile<2, T2>
+                                 : k_nl_build<2, T2, false>;
+  SPH_LAUNCH(ws, "skin_build", st, (kernel<<<build_grid(ws, tile), kBlock, 0, st>>>(a)));
   return SPH_OK;
 }
 
 // What a skin build leaves to reduce: the largest list of one particle ->
 // info[7] (only on a rebuild).
 Reduce skin_build_tail(sph_ws* ws, int64_t* info) {
-  const int blocks = (int)xcd_grid(cdiv((int64_t)ws->cfg.n * ws->tpp, kBlock), ws->xcd_remap);
+  const int blocks = (int)build_grid(ws, skin_tiled(ws->cfg));
   return Reduce{ws->part_build, blocks, nullptr, &info[7], info, -1, ws->sk.flag, nullptr};
 }
 
@@ -1598,12 +1979,18 @@ __global__ __launch_bounds__(256) void k_cell_sort_ens(const EnsBin* __restrict_
                       a.g, a.cell_count);
 }
 
+// The members of a 2D ensemble are many particles together, where the lanes'
+// build is the faster one (see tiled()).
 template <int DIM, int TPP>
 __global__ __launch_bounds__(kBlock, 6) void k_nl_build_ens(const BuildArgs* __restrict__ t,
-                                                         const EnsBlock* __restrict__ map) {
+                                                            const EnsBlock* __restrict__ map) {
   const EnsBlock m = map[blockIdx.x];
   if (m.sim < 0) return;
-  nl_build_body<DIM, TPP, false, false>(t[m.sim], m.blk);
+  // a block of the map is kBlock / TPP particles
+  if constexpr (DIM == 3)
+    nl_tile_body<DIM, TPP>((ColdArgs*)(t + m.sim), m.blk, kBlock / TPP);
+  else
+    nl_build_body<DIM, TPP, false>(t[m.sim], m.blk);
 }
 
 // one workgroup per member

@@ -118,8 +118,12 @@ extern "C" int sph_ws_create(const sph_nl_config* cfg, sph_ws** out) {
   A(ws->off64, N + 1);
   A(ws->scan_tmp, 1024);
   A(ws->cnt_id, N);
-  // workgroups of the widest launch (npad * tpp lanes of 256, rounded to 8 XCDs)
-  ws->part_blocks = (int32_t)(((npad * ws->tpp + 255) / 256 + 7) / 8 * 8);
+  // workgroups of the widest launch (npad * tpp lanes of 256, or tile_range
+  // particles each; rounded to 8 XCDs)
+  const int64_t sweep_blocks = (npad * ws->tpp + 255) / 256;
+  const int64_t range = tile_range(cfg->dim, N), tile_blocks = (N + range - 1) / range;
+  ws->part_blocks =
+      (int32_t)(((sweep_blocks > tile_blocks ? sweep_blocks : tile_blocks) + 7) / 8 * 8);
   A(ws->part_build, 2 * (int64_t)ws->part_blocks);
   A(ws->part_sweep, 2 * (int64_t)ws->part_blocks);
   for (int b = 0; b < 2; ++b) {
@@ -206,7 +210,7 @@ extern "C" int sph_skin_enable(sph_ws* ws, float skin, int32_t width) {
   A(S.b.cell_start, ncell + 1);
   A(S.b.ell, ws->tpp * lw * npad);
   A(S.b.cnt, ws->tpp * npad);
-  A(S.b.pos, N + kSkinPosPad);  // last, so that its padding moves no other buffer
+  A(S.b.pos, N);
 #undef A
   if (rc == SPH_OK) {
     const int32_t one = 1;  // the first step builds the lists
