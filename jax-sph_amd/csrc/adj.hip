@@ -96,7 +96,9 @@ __device__ __forceinline__ bool bc_holds(int kind, int tag) {
   return false;
 }
 
-template <int DIM, bool TVF>
+// SCALED (k_adj_forces): la = abar' / m and lb = p_bg bbar' / m, the l and n of
+// the pair differences; else the cotangents as they are.
+template <int DIM, bool TVF, bool SCALED>
 __global__ void k_adj_gather(AdjArgs a) {
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= a.s.n) return;
@@ -104,8 +106,15 @@ __global__ void k_adj_gather(AdjArgs a) {
   // the hook replaces the accelerations of the particles it holds
   const bool held = bc_holds(a.bc_kind, a.s.in.tag[i]);
   const V3 zero = {0.f, 0.f, 0.f};
-  a.la[s] = f4(held ? zero : load_vec<DIM>(a.ab_in, i), 0.0f);
-  if (TVF) a.lb[s] = f4(held || !a.bb_in ? zero : load_vec<DIM>(a.bb_in, i), 0.0f);
+  V3 la = held ? zero : load_vec<DIM>(a.ab_in, i);
+  V3 lb = !TVF || held || !a.bb_in ? zero : load_vec<DIM>(a.bb_in, i);
+  if (SCALED) {
+    const float inv_m = 1.0f / a.s.in.mass[i];
+    la = inv_m * la;
+    lb = (make_eos(a.s.prm).p_fn(0.0f) * inv_m) * lb;
+  }
+  a.la[s] = f4(la, 0.0f);
+  if (TVF) a.lb[s] = f4(lb, 0.0f);
 }
 
 // Sweep A: density cotangent (times m, fluid only), the u' and v' cotangents
@@ -123,6 +132,14 @@ __global__ void k_adj_gather(AdjArgs a) {
 //   a_k += C m_j psi_kj (du . r_kj) r_kj for fluid j,  psi = W'(d) / (rho_k rho_j d^3),
 // C = alpha h c_ref rho_ref; the same transpose with l = m_j [j fluid] abar'_k -
 // m_k [k fluid] abar'_j, and d psi / d rho_k = -psi / rho_k.
+// Bound by VALU issue and the gathers, then by the memory the lists and records
+// come from (a rollout's steps are beyond the caches): 110,592 3D particles
+// with transport velocity 114 us with l and n differenced per use and six
+// records a pair, 103 us with l = abar'/m, n = p_bg bbar'/m scaled beforehand,
+// the sums' common factors applied once, and v - u and p from one record (the
+// viscosity and tag only where needed), 95 us with the indices further ahead;
+// 10,000 2D particles 14.1 and 12.2.  A bound on the registers costs more in
+// spills than it gains in wavefronts (6 waves a SIMD: 134 us).
 template <int DIM, int KIND, bool TVF, bool WALLS, bool CONT, bool AV>
 __global__ __launch_bounds__(kAB) void k_adj_forces(AdjArgs aa, float4* __restrict__ ab0,
                                                     float4* __restrict__ ab1,
@@ -137,32 +154,39 @@ __global__ __launch_bounds__(kAB) void k_adj_forces(AdjArgs aa, float4* __restri
   const Eos eos = make_eos(p);
   const float4* __restrict__ RU = WALLS ? a.R.U2 : a.R.U1;
   const float4* __restrict__ RQ = WALLS ? a.R.Q2 : a.R.Q1;
-  const float4* __restrict__ RV = WALLS ? a.R.V2 : a.R.V0;
-  const float4 Pk = a.R.P[k], Uk = RU[k], Qk = RQ[k], Lk4 = aa.la[k];
+  const float4* __restrict__ RW = WALLS ? a.R.W2 : a.R.W1;  // (v - u, p)
+  const float4 Pk = a.R.P[k], Uk = RU[k], Qk = RQ[k];
   const float mk = Pk.w, rhok = Uk.w, pk = Qk.x, etak = Qk.y;
   const float Vk2 = (mk / rhok) * (mk / rhok);
+  const float cVk = -2.0f * Vk2 / rhok;  // d V_k^2 / d rho_k
+  const float hrhok = 0.5f * rhok;
   const float dPk = eos.dp_drho(rhok);
-  const float inv_mk = 1.0f / mk;
-  const V3 uk = v3(Uk), lk = v3(Lk4);
-  // transport-velocity terms: w = v - u, the background pressure of G and the
-  // sorted cotangent of b'
-  const V3 wk = TVF ? v3(RV[k]) - uk : V3{0.f, 0.f, 0.f};
+  const V3 uk = v3(Uk), lk = v3(aa.la[k]);
+  // transport-velocity terms: w = v - u and the scaled cotangent of b'
+  const V3 wk = TVF ? v3(RW[k]) : V3{0.f, 0.f, 0.f};
   const V3 nk = TVF ? v3(aa.lb[k]) : V3{0.f, 0.f, 0.f};
-  const float pbg = TVF ? eos.p_fn(0.0f) : 0.0f;
   const bool fluid = (int)Qk.z == kFluid;
   const float avK = AV ? p.artificial_alpha * p.av_h * 10.0f : 0.0f;  // alpha h c_ab
   const float av_h2 = AV ? 0.01f * p.av_h * p.av_h : 0.0f;
   const float dK = p.solver == 2 ? p.diff_alpha * p.support * p.c_ref * p.rho_ref : 0.0f;
-  float rhob = 0.0f;
+  // the tag and viscosity of j are read where they are needed: for the terms
+  // of fluid pairs, or if viscosities differ (else eta_kj is particle k's own)
+  const bool need_q = AV || dK != 0.0f || *a.eta_varies != 0;
+  const float eta_kk = 2.0f * etak * etak * rcp_fast(etak + etak + kEps);
+  float rhob = 0.0f, sul = 0.0f;
   V3 ub = {0.f, 0.f, 0.f}, rb = {0.f, 0.f, 0.f}, vb = {0.f, 0.f, 0.f};
-  for_each_pair(a, k, h, [&](const int j) {
-    const float4 Pj = a.R.P[j];
+  struct Rec { float4 P; };
+  const auto load = [&](const int j) { Rec r; r.P = a.R.P[j]; return r; };
+  for_each_pair_far<4>(a, k, h, load, [&](const int j, const Rec& rr) {
+    const float4 Pj = rr.P;
     const V3 dr = min_image<DIM>(Pk, Pj, a.geo);
     const float d2 = dist2<DIM>(dr.x, dr.y, dr.z);
     if (d2 == 0.0f) return;  // self pair: every term and derivative vanishes
     if (!in_cutoff<DIM>(a, d2, Pk, Pj)) return;
-    const float4 Uj = RU[j], Qj = RQ[j], Lj4 = aa.la[j];
-    const float mj = Pj.w, rhoj = Uj.w, pj = Qj.x, etaj = Qj.y;
+    const float4 Uj = RU[j], Wj = RW[j], Lj4 = aa.la[j];
+    float4 Qj = make_float4(0.0f, etak, 0.0f, 0.0f);
+    if (need_q) Qj = RQ[j];
+    const float mj = Pj.w, rhoj = Uj.w, pj = Wj.w, etaj = Qj.y;
     // hardware rsqrt/rcp (about 1 ulp), as in the forward sweeps; 1/(d + eps)
     // is 1/d in float32 for every d above ~4e-9 (eps = 2.2e-16)
     const float inv = rsq_fast(d2);
@@ -171,46 +195,39 @@ __global__ __launch_bounds__(kAB) void k_adj_forces(AdjArgs aa, float4* __restri
     const float w1 = K.dw(q);
     const float w2 = K.d2w(q);
     const float A0 = w1 * inv;                      // W'(d) / (d + eps)
-    const float Ad0 = (w2 - w1 * inv) * inv;        // d/dd of the above
-    const float inv_mj = rcp_fast(mj);
-    const float Akj = A0 * inv_mk, Ajk = A0 * inv_mj;
-    const float Adkj = Ad0 * inv_mk, Adjk = Ad0 * inv_mj;
+    const float Ad0 = (w2 - A0) * inv;              // d/dd of the above
     const float Vj = mj * rcp_fast(rhoj);
-    const float Vj2 = Vj * Vj;
-    const float Vs = Vk2 + Vj2;
+    const float Vs = Vk2 + Vj * Vj;
+    const float g = Vs * A0;
     const float rs = rhok + rhoj;
     const float irs = rcp_fast(rs);
     const float pkj = (rhoj * pk + rhok * pj) * irs;
-    const float etakj = 2.0f * etak * etaj * rcp_fast(etak + etaj + kEps);
-    const V3 uj = v3(Uj);
-    V3 T = (-pkj) * dr + etakj * (uk - uj);
-    V3 wj = {0.f, 0.f, 0.f};
-    if (TVF) {
-      wj = v3(RV[j]) - uj;
-      T = T + (0.5f * rhok * dot<DIM>(wk, dr)) * uk + (0.5f * rhoj * dot<DIM>(wj, dr)) * uj;
-    }
+    float etakj = eta_kk;
+    if (need_q) etakj = 2.0f * etak * etaj * rcp_fast(etak + etaj + kEps);
     const float Dp = rhoj * (dPk * rs + (pj - pk)) * (irs * irs);  // d p_kj / d rho_k (via p_k)
-    const V3 lj = v3(Lj4);
-    const V3 lA = Akj * lk - Ajk * lj;   // W'/(d + eps) l_kj
-    const V3 lc = Vs * lA;               // (V_k^2 + V_j^2) W'/(d + eps) l_kj
-    const V3 lAd = Adkj * lk - Adjk * lj;
-    rhob += (-2.0f * Vk2 / rhok) * dot<DIM>(lA, T) - Dp * dot<DIM>(lc, dr);
-    ub = ub + etakj * lc;
-    rb = rb + Vs * ((dot<DIM>(lAd, T) * inv) * dr - pkj * lA);
+    const V3 uj = v3(Uj);
+    // l_kj, and l_kj . T_kj with T taken apart; E adds p_bg n_kj . r_kj
+    const V3 l = lk - v3(Lj4);
+    const float lr = dot<DIM>(l, dr);
+    float E = etakj * dot<DIM>(l, uk - uj) - pkj * lr;
+    float eta_a = etakj;  // coefficient of g l in ub
     if (TVF) {
-      const V3 nj = v3(aa.lb[j]);
-      const V3 nA = Akj * nk - Ajk * nj;     // W'/(d + eps) n_kj
-      const V3 nAd = Adkj * nk - Adjk * nj;
-      const float uk_lc = dot<DIM>(uk, lc), wk_r = dot<DIM>(wk, dr);
-      // G: the volume factor and the pair geometry
-      rhob += (-2.0f * Vk2 / rhok) * pbg * dot<DIM>(nA, dr);
-      rb = rb + (Vs * pbg) * ((dot<DIM>(nAd, dr) * inv) * dr + nA);
+      const V3 wj = v3(Wj), n = nk - v3(aa.lb[j]);
+      const float luk = dot<DIM>(l, uk), luj = dot<DIM>(l, uj);
+      const float wkr = dot<DIM>(wk, dr), hrhoj = 0.5f * rhoj;
+      const float ak = hrhok * wkr;
+      E += ak * luk + (hrhoj * dot<DIM>(wj, dr)) * luj + dot<DIM>(n, dr);
+      eta_a += ak;
       // the stress A_k = rho_k u_k w_k^T of T: through rho_k, u_k, v_k and r
-      rhob += 0.5f * wk_r * uk_lc;
-      ub = ub + (0.5f * rhok) * (wk_r * lc - uk_lc * dr);
-      vb = vb + (0.5f * rhok * uk_lc) * dr;
-      rb = rb + (0.5f * rhok * uk_lc) * wk + (0.5f * rhoj * dot<DIM>(uj, lc)) * wj;
+      const float ul = g * luk;
+      sul += ul;
+      rhob += 0.5f * wkr * ul;
+      vb = vb + ul * dr;  // times rho_k / 2 after the sum; ub takes its negative
+      rb = rb + g * n + (hrhoj * (g * luj)) * wj;
     }
+    rhob += cVk * (A0 * E) - Dp * (g * lr);
+    ub = ub + (eta_a * g) * l;
+    rb = rb + (Vs * Ad0 * inv * E) * dr - (g * pkj) * l;
     if (AV && fluid && (int)Qj.z == kFluid) {
       const float D = d2 + av_h2;
       const float iD = rcp_fast(D);
@@ -218,13 +235,13 @@ __global__ __launch_bounds__(kAB) void k_adj_forces(AdjArgs aa, float4* __restri
       const float Kphi = avK * A0 * irab * iD;    // K phi
       const V3 du = uk - uj;
       const float e = dot<DIM>(du, dr);
-      const V3 l = mj * lk - mk * lj;
-      const float sl = dot<DIM>(dr, l);
+      const V3 lav = (mj * mk) * l;
+      const float sl = (mj * mk) * lr;
       // d phi / dd, over d
       const float dphi = (Ad0 * D - 2.0f * A0 * d) * irab * iD * iD * inv;
       ub = ub + (Kphi * sl) * dr;
       rhob -= Kphi * e * sl * irs;                // d phi / d rho_k = -phi / (rho_k + rho_j)
-      rb = rb + (avK * dphi * e * sl) * dr + Kphi * (sl * du + e * l);
+      rb = rb + (avK * dphi * e * sl) * dr + Kphi * (sl * du + e * lav);
     }
     const bool fluid_j = (int)Qj.z == kFluid;
     if (dK != 0.0f && (fluid || fluid_j)) {
@@ -233,14 +250,20 @@ __global__ __launch_bounds__(kAB) void k_adj_forces(AdjArgs aa, float4* __restri
       const float dpsi = (Ad0 * d - 2.0f * A0) * (inv * inv) * (inv * inv) * ipp;  // psi' / d
       const V3 du = uk - uj;
       const float e = dot<DIM>(du, dr);
-      const V3 l = (fluid_j ? mj : 0.0f) * lk - (fluid ? mk : 0.0f) * lj;
-      const float sl = dot<DIM>(dr, l);
+      const float mm = mj * mk;
+      const V3 ld = (fluid_j ? mm : 0.0f) * lk - (fluid ? mm : 0.0f) * v3(Lj4);
+      const float sl = dot<DIM>(dr, ld);
       const float Kpsi = dK * psi;
       ub = ub + (Kpsi * sl) * dr;
       rhob -= Kpsi * e * sl / rhok;
-      rb = rb + (dK * dpsi * e * sl) * dr + Kpsi * (sl * du + e * l);
+      rb = rb + (dK * dpsi * e * sl) * dr + Kpsi * (sl * du + e * ld);
     }
   });
+  if (TVF) {
+    vb = hrhok * vb;
+    ub = ub - vb;
+    rb = rb + (hrhok * sul) * wk;
+  }
   rhob = lane_sum<TPP>(rhob);
   ub = lane_sum<TPP>(ub);
   rb = lane_sum<TPP>(rb);
@@ -1041,7 +1064,7 @@ int launch_adjoint_rie(sph_ws* ws, AdjArgs& a, bool records_ready, hipStream_t s
     SPH_LAUNCH(ws, "density", st,
                (k_density<DIM, KIND, CONT ? 2 : 0><<<grid, kAB, 0, st>>>(a.s)));
   SPH_LAUNCH(ws, "adj_gather", st,
-             (k_adj_gather<DIM, TVF><<<(unsigned)cdivl(n, kAB), kAB, 0, st>>>(a)));
+             (k_adj_gather<DIM, TVF, false><<<(unsigned)cdivl(n, kAB), kAB, 0, st>>>(a)));
   SPH_LAUNCH(ws, "adj_forces", st,
              (k_adj_forces_rie<DIM, KIND, AV, CONT, TVF><<<grid, kAB, 0, st>>>(
                  a, ws->AB0, ws->AB1, ws->DL0)));
@@ -1075,7 +1098,7 @@ int launch_adjoint(sph_ws* ws, AdjArgs& a, bool records_ready, hipStream_t st) {
     if (WALLS) SPH_LAUNCH(ws, "walls", st, (k_walls<DIM, KIND, 0><<<grid, kAB, 0, st>>>(a.s)));
   }
   SPH_LAUNCH(ws, "adj_gather", st,
-             (k_adj_gather<DIM, TVF><<<(unsigned)cdivl(n, kAB), kAB, 0, st>>>(a)));
+             (k_adj_gather<DIM, TVF, true><<<(unsigned)cdivl(n, kAB), kAB, 0, st>>>(a)));
   SPH_LAUNCH(ws, "adj_forces", st,
              (k_adj_forces<DIM, KIND, TVF, WALLS, CONT, AV><<<grid, kAB, 0, st>>>(
                  a, ws->AB0, ws->AB1, ws->AB2)));
@@ -1191,6 +1214,7 @@ extern "C" int sph_step_vjp(sph_ws* ws, int bank, const sph_solver_params* prm, 
     // force and wall sweeps do); rho_c keeps the continuity density
     a.s.R.U1 = ws->U3;
     a.s.R.Q1 = ws->Q3;
+    a.s.R.W1 = ws->W3;
   }
   a.dt = dt;
   a.c_tvf = tvf_coef;

@@ -244,6 +244,38 @@ __device__ __forceinline__ void for_each_pair_ahead(const SweepArgs& a, int s, i
   }
 }
 
+// for_each_pair_ahead with the indices requested D pairs before their records,
+// for a sweep whose lists come from memory and not from a cache (the transposes
+// of a rollout that keeps every step's list): k_adj_forces of 110,592 particles
+// 103 us with D = 1, 97 with 2, 95 with 4, 93 with 6.  The forward sweeps read
+// lists just built and gain nothing.
+template <int D, typename L, typename F>
+__device__ __forceinline__ void for_each_pair_far(const SweepArgs& a, int s, int h, L&& load,
+                                                  F&& f) {
+  const int c = a.cnt[h * a.npad + s];
+  if (c <= 0) return;
+  const int32_t* lst = a.ell + ((int64_t)h * a.lane_width) * a.npad + s;
+  int next[D];  // indices of pairs k + 1 ...
+  int j = lst[0];
+#pragma unroll
+  for (int q = 0; q < D; ++q) next[q] = q + 1 < c ? lst[(int64_t)(q + 1) * a.npad] : j;
+  const int32_t* far = lst + (int64_t)(D + 1) * a.npad;
+  __builtin_assume(j >= 0);
+  auto rec = load(j);
+  for (int k = 0; k < c; ++k) {
+    const int jc = j;
+    const auto rc = rec;
+    j = next[0];
+    __builtin_assume(j >= 0);
+#pragma unroll
+    for (int q = 0; q + 1 < D; ++q) next[q] = next[q + 1];
+    if (k + D + 1 < c) next[D - 1] = *far;
+    far += a.npad;
+    rec = load(j);
+    f(jc, rc);
+  }
+}
+
 // Sum of x over the TPP consecutive lanes serving one particle.
 template <int TPP>
 __device__ __forceinline__ float lane_sum(float x) {
