@@ -183,7 +183,9 @@ __global__ __launch_bounds__(kAB) void k_adj_forces(AdjArgs aa, float4* __restri
     const float d2 = dist2<DIM>(dr.x, dr.y, dr.z);
     if (d2 == 0.0f) return;  // self pair: every term and derivative vanishes
     if (!in_cutoff<DIM>(a, d2, Pk, Pj)) return;
-    const float4 Uj = RU[j], Wj = RW[j], Lj4 = aa.la[j];
+    const float4 Uj = RU[j], Lj4 = aa.la[j];
+    float4 Wj = make_float4(0.0f, 0.0f, 0.0f, Uj.z);  // 2D without w: p beside u
+    if (TVF || DIM == 3) Wj = RW[j];
     float4 Qj = make_float4(0.0f, etak, 0.0f, 0.0f);
     if (need_q) Qj = RQ[j];
     const float mj = Pj.w, rhoj = Uj.w, pj = Wj.w, etaj = Qj.y;

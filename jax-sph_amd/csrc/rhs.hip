@@ -176,7 +176,7 @@ __device__ __forceinline__ void renorm_run(const SweepArgs& a, const int blk) {
   const float4 Ui = a.R.U1[s], Qi = a.R.Q1[s];
   const float pr = eos.p_fn(rho);
   const float4 Vi = a.R.V0[s];
-  a.R.U3[s] = make_float4(Ui.x, Ui.y, Ui.z, rho);
+  a.R.U3[s] = u_record<DIM>(v3(Ui), rho, pr);
   a.R.Q3[s] = make_float4(pr, Qi.y, Qi.z, Qi.w);
   a.R.W3[s] = make_float4(Vi.x - Ui.x, Vi.y - Ui.y, Vi.z - Ui.z, pr);
 }
@@ -244,8 +244,9 @@ __device__ __forceinline__ void force_run(const SweepArgs& a, const int blk) {
     const float4 Uj = a.Uf[j];
     float4 Qj = make_float4(0.0f, etai, 0.0f, 0.0f);
     if (need_q) Qj = a.Qf[j];
-    float4 Wj = make_float4(0.0f, 0.0f, 0.0f, Qj.x);  // (v - u, p) of j
-    if (SOLVER != 1 && (TVF || !need_q)) Wj = a.Wf[j];
+    // (v - u, p) of j; without the stress only p, which 2D has beside u
+    float4 Wj = make_float4(0.0f, 0.0f, 0.0f, DIM == 2 ? Uj.z : Qj.x);
+    if (SOLVER != 1 && (TVF || (DIM == 3 && !need_q))) Wj = a.Wf[j];
     const float mj = Pj.w, rhoj = Uj.w, pj = Wj.w, etaj = Qj.y;
     const V3 uj = v3(Uj);
     const float Vj = mj * rcp_fast(rhoj);
