@@ -410,8 +410,11 @@ class GraphRollout:
             gV = torch.cuda.CUDAGraph()
             with torch.cuda.graph(gV):
                 cur = dict(self.bar)
-                for st_j, nb_j in reversed(steps):
-                    out = {key: torch.empty_like(v) for key, v in cur.items()}
+                for j, (st_j, nb_j) in reversed(list(enumerate(steps))):
+                    # the segment's last transpose leaves its cotangents where the
+                    # next segment's reads them (never where it reads its own)
+                    out = self.bar if j == 0 and self.k > 1 else \
+                        {key: torch.empty_like(v) for key, v in cur.items()}
                     bar_in = _cot_in(cur)
                     bar_out = _cot_out(out)
                     _lib.check(L.sph_step_vjp(nb_j.workspace.handle, nb_j.bank,
@@ -422,8 +425,9 @@ class GraphRollout:
                                               1,  # records left by this step's own R pass
                                               _lib.stream()), "sph_step_vjp")
                     cur = out
-                for key, dst in self.bar.items():
-                    dst.copy_(cur[key])
+                if cur is not self.bar:
+                    for key, dst in self.bar.items():
+                        dst.copy_(cur[key])
             self.gR.append(gR)
             self.gV.append(gV)
             self._steps.append(steps)   # keeps the recomputed states alive

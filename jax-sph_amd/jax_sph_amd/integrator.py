@@ -61,17 +61,20 @@ def si_euler(tvf: float, model: Callable, shift_fn: Callable, bc_fn: Callable,
             return None
         return _bc_spec(bc_fn)
 
-    def _fused(dt, state, neighbors, spec):
+    def _fused(dt, state, neighbors, spec, out=None, info=None):
+        # out, info (or None: new ones): buffers of a captured graph for the
+        # step's results other than the positions, and for its error block
         ws = neighbors.workspace
         neighbors._check_live()
         s = solver.state_in(state)
         if s["r"].shape[0] != ws.n:
             raise ValueError("state size does not match the neighbour list")
-        out = solver.new_outputs(s)
+        out = solver.new_outputs(s) if out is None else out
         r_out = torch.empty_like(s["r"])
         bank = neighbors._search.step_bank(neighbors)
         ws.generation[bank] += 1
-        info = torch.empty(8, dtype=torch.int64, device=r_out.device)
+        if info is None:
+            info = torch.empty(8, dtype=torch.int64, device=r_out.device)
         dtf = _f(dt)
         ctvf = _f(_f(tvf * 0.5) * dtf)
         # v == u exactly when tvf == 0, so the A = rho u (v-u) stress vanishes
@@ -123,6 +126,7 @@ def si_euler(tvf: float, model: Callable, shift_fn: Callable, bc_fn: Callable,
         return state, neighbors
 
     advance._sph_fusable = _fusable
+    advance._sph_fused = _fused
     # what an ensemble needs to issue this step itself (see ensemble.py)
     advance._sph_solver = solver
     advance._sph_tvf = tvf

@@ -166,13 +166,13 @@ class WCSPH:
         g = self.g_ext_fn(r)
         return _lib.as_f32(g)
 
+    def output_keys(self):
+        """The fields a right-hand side writes."""
+        keys = ("u", "v", "dudt", "dvdt", "rho", "p", "drhodt")
+        return keys + ("T", "dTdt") if self.is_heat_conduction else keys
+
     def new_outputs(self, s):
-        out = {k: torch.empty_like(s[k]) for k in ("u", "v", "dudt", "dvdt", "rho", "p",
-                                                   "drhodt")}
-        if self.is_heat_conduction:
-            out["T"] = torch.empty_like(s["T"])
-            out["dTdt"] = torch.empty_like(s["dTdt"])
-        return out
+        return {k: torch.empty_like(s[k]) for k in self.output_keys()}
 
     @staticmethod
     def c_state_out(out) -> _lib.StateOut:
