@@ -537,7 +537,7 @@ int launch_kind(sph_ws* ws, SweepArgs& a, const Reduce& on_density, const Reduce
   return for_plan_kind<DIM>(pl, [&](const char* name, SweepKernel k, EnsSweepKernel) -> int {
     const bool density = !std::strcmp(name, "density"), force = !std::strcmp(name, "force");
     a.tail = density ? on_density : force ? on_force : Reduce{};
-    const unsigned grid = blocks + (a.tail.part ? 1 : 0);
+    const unsigned grid = blocks + (a.tail.part ? kTailBlocks : 0);
     SPH_LAUNCH(ws, name, st, (k<<<grid, kB, 0, st>>>(a)));
     return 0;
   });

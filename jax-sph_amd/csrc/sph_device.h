@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include "../../include/sph.h"
+#include "block_map.h"
 
 namespace sph {
 
@@ -262,23 +263,8 @@ __device__ __forceinline__ Eos make_eos(const sph_solver_params& p) {
   return e;
 }
 
-// ------------------------------------------------------------ XCD mapping
-// MI355X dispatches the workgroups of a launch to its 8 XCDs round-robin by
-// workgroup id, and each XCD has its own L2.  With remap on (and a grid that
-// is a multiple of 8), XCD x runs the contiguous logical blocks
-// [x * per, (x + 1) * per): cell-sorted particles that share neighbours then
-// share one L2 instead of being spread over all eight.
-constexpr int kXcds = 8;
-__device__ __forceinline__ int logical_block_of(int b, int blocks, int remap) {
-  if (!remap) return b;
-  const int per = blocks / kXcds;
-  return (b % kXcds) * per + b / kXcds;
-}
 __device__ __forceinline__ int logical_block(int remap) {
   return logical_block_of(blockIdx.x, gridDim.x, remap);
-}
-__host__ __device__ inline unsigned xcd_grid(long long blocks, int remap) {
-  return (unsigned)(remap ? (blocks + kXcds - 1) / kXcds * kXcds : blocks);
 }
 
 // Batched launches over the members of an ensemble: workgroup b of the launch

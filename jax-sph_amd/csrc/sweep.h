@@ -195,9 +195,9 @@ struct SweepArgs {
   int64_t* info;  // non-null: the density sweep counts pairs (per-workgroup partials in part)
   int64_t* part;  // [2 * gridDim.x] pairs and largest list of each workgroup
   int remap;      // XCD-contiguous block order (grid a multiple of 8)
-  // tail.part non-null: the launch has one workgroup more, its first, which
-  // reduces the partials of an earlier launch (a launch of its own costs the
-  // stream 4-5 us, and nothing of this sweep reads the result)
+  // tail.part non-null: the launch's first workgroup reduces the partials of
+  // an earlier launch (a launch of its own costs the stream 4-5 us, and nothing
+  // of this sweep reads the result); kTailBlocks more than the sweep's own
   Reduce tail;
 };
 
@@ -356,13 +356,12 @@ __global__ void k_gather_state(SweepArgs a, const float* __restrict__ r, const f
 #define SPH_SWEEP_KERNELS(NAME, RUN, TPARAMS, TARGS, MINW)                                \
   template <SPH_UNPAREN TPARAMS>                                                          \
   __global__ __launch_bounds__(kB, MINW) void NAME(SweepArgs a) {                         \
-    const int extra = a.tail.part != nullptr;                                             \
-    if (extra && blockIdx.x == 0) {                                                       \
-      reduce_parts_body<kB>(a.tail);                                                      \
+    const bool tail = a.tail.part != nullptr;                                             \
+    if (tail && (int)blockIdx.x < kTailBlocks) {                                          \
+      if (blockIdx.x == 0) reduce_parts_body<kB>(a.tail);                                 \
       return;                                                                             \
     }                                                                                     \
-    RUN<SPH_UNPAREN TARGS>(a, logical_block_of(blockIdx.x - extra, gridDim.x - extra,     \
-                                               a.remap));                                 \
+    RUN<SPH_UNPAREN TARGS>(a, sweep_block_of(blockIdx.x, gridDim.x, tail, a.remap));      \
   }                                                                                       \
   template <SPH_UNPAREN TPARAMS>                                                          \
   __global__ __launch_bounds__(kB, MINW) void NAME##_ens(const SweepArgs* __restrict__ t, \
