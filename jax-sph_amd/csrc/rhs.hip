@@ -196,7 +196,10 @@ __device__ __forceinline__ void force_run(const SweepArgs& a, const int blk) {
   constexpr int TPP = tpp_of(DIM);
   const int tid = blk * blockDim.x + threadIdx.x;
   const int s = tid / TPP, h = tid % TPP;
-  if (s >= a.n) return;  // whole lane groups leave together
+  if (s >= a.n) {  // whole lane groups leave together
+    if (tail_block(a)) reduce_parts_body<kB>(a.tail);
+    return;
+  }
   const sph_solver_params& p = a.prm;
   const KernelEval<KIND, DIM> K{p.kernel, p.sigma, p.one_over_h};
   const Eos eos = make_eos(p);

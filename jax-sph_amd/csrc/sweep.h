@@ -201,6 +201,19 @@ struct SweepArgs {
   Reduce tail;
 };
 
+// The workgroup that reduces for an earlier launch.  The sweeps look for it
+// where threads without a particle leave anyway: a branch before the sweep
+// costs its loop registers (the 3D standard force with transport velocity,
+// which fills its 64, went to scratch memory: 1,566 us at 128^3, without the
+// branch 1,557; the delta-SPH force with artificial viscosity lost a wavefront
+// a SIMD: 178 us at 64^3, without 170).
+__device__ __forceinline__ bool tail_block(const SweepArgs& a) {
+  return a.tail.part != nullptr && blockIdx.x == 0;
+}
+__device__ __forceinline__ int sweep_block(const SweepArgs& a) {
+  return sweep_block_of(blockIdx.x, gridDim.x, a.tail.part != nullptr, a.remap);
+}
+
 // Pair (sweep centre s, listed j) of the neighbour set: the reference predicate
 // metric_sq(r_s, r_j) < cutoff^2 with s in the sender role, as in the build.
 template <int DIM>
@@ -356,12 +369,7 @@ __global__ void k_gather_state(SweepArgs a, const float* __restrict__ r, const f
 #define SPH_SWEEP_KERNELS(NAME, RUN, TPARAMS, TARGS, MINW)                                \
   template <SPH_UNPAREN TPARAMS>                                                          \
   __global__ __launch_bounds__(kB, MINW) void NAME(SweepArgs a) {                         \
-    const bool tail = a.tail.part != nullptr;                                             \
-    if (tail && (int)blockIdx.x < kTailBlocks) {                                          \
-      if (blockIdx.x == 0) reduce_parts_body<kB>(a.tail);                                 \
-      return;                                                                             \
-    }                                                                                     \
-    RUN<SPH_UNPAREN TARGS>(a, sweep_block_of(blockIdx.x, gridDim.x, tail, a.remap));      \
+    RUN<SPH_UNPAREN TARGS>(a, sweep_block(a));                                            \
   }                                                                                       \
   template <SPH_UNPAREN TPARAMS>                                                          \
   __global__ __launch_bounds__(kB, MINW) void NAME##_ens(const SweepArgs* __restrict__ t, \
@@ -535,6 +543,10 @@ __device__ __forceinline__ int density_of(const SweepArgs& a, const int s, const
 // workgroup's partials.
 template <int DIM, int KIND, int MODE>
 __device__ __forceinline__ void density_run(const SweepArgs& a, const int blk) {
+  if (a.tail.part && (int)blockIdx.x < kTailBlocks) {
+    if (blockIdx.x == 0) reduce_parts_body<kB>(a.tail);
+    return;
+  }
   constexpr int TPP = tpp_of(DIM);
   const int tid = blk * blockDim.x + threadIdx.x;
   const int s = tid / TPP, h = tid % TPP;
