@@ -200,10 +200,14 @@ extern "C" int sph_ensemble_step(sph_ensemble* e, hipStream_t st) {
     set_error("sph_ensemble_step: null ensemble");
     return SPH_ERR_ARG;
   }
-  for (auto& m : e->m) m.ws->sk.stepped = true;
+  int rc = SPH_OK;
+  for (auto& m : e->m) {
+    m.ws->sk.stepped = true;
+    if (!rc) rc = clean_histograms(m.ws, st);
+  }
   sph_ws* prof = e->m[0].ws;
   // 1. kick/drift + rebuild test + reference-grid occupancy; skin binning where needed
-  int rc = ens_skin_begin(e->nl, e->dim, e->part, e->cells, prof, st);
+  if (!rc) rc = ens_skin_begin(e->nl, e->dim, e->part, e->cells, prof, st);
   // 2. sorted records (and build positions), then the lists of members that rebuild
   if (!rc) rc = ens_gather(e->rhs, e->dim, e->part, prof, st);
   if (!rc) rc = ens_skin_build(e->nl, e->dim, e->lanes, prof, st);
@@ -212,6 +216,8 @@ extern "C" int sph_ensemble_step(sph_ensemble* e, hipStream_t st) {
     if (!rc) rc = ens_sweeps(e->rhs, e->dim, g.plan, g.lanes, prof, st);
   // 4. occupancy, largest list, overflow bit; rebuild requests consumed
   if (!rc) rc = ens_skin_finish(e->nl, prof, st);
+  if (rc)
+    for (auto& m : e->m) HistogramGuard{m.ws, st};
   return rc;
 }
 

@@ -13,6 +13,7 @@
 #include <mutex>
 #include <string>
 #include <type_traits>
+#include <vector>
 
 #include "ens.h"
 #include "sph_device.h"
@@ -30,6 +31,25 @@ template <typename T>
 __global__ void k_fill(T* __restrict__ a, int64_t n, T v) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) a[i] = v;
+}
+
+static hipError_t clear_counts(int32_t* count, int64_t ncell, bool* dirty, hipStream_t st) {
+  if (!*dirty) return hipSuccess;
+  k_fill<int32_t><<<cdiv(ncell, kBlock), kBlock, 0, st>>>(count, ncell, 0);
+  const hipError_t e = hipGetLastError();
+  *dirty = e != hipSuccess;
+  return e;
+}
+
+int clean_histograms(sph_ws* ws, hipStream_t st) {
+  hipError_t e = clear_counts(ws->cell_count, ws->ncell, &ws->count_dirty, st);
+  if (e == hipSuccess) e = clear_counts(ws->sk.cell_count, ws->sk.ncell, &ws->sk.count_dirty, st);
+  return e == hipSuccess ? SPH_OK : hip_fail(e, "clean_histograms");
+}
+
+HistogramGuard::~HistogramGuard() {
+  (void)clear_counts(ws->cell_count, ws->ncell, &ws->count_dirty, s);
+  (void)clear_counts(ws->sk.cell_count, ws->sk.ncell, &ws->sk.count_dirty, s);
 }
 
 struct Grid {
@@ -1564,7 +1584,9 @@ int integrate_and_hash(sph_ws* ws, const float* r, const float* u, const float* 
   const auto& c = ws->cfg;
   const int n = c.n;
   Grid g = make_grid(c);
-  const auto kernel = bins_small(n, ws->ncell)
+  const bool small = bins_small(n, ws->ncell);
+  ws->count_dirty = !small;
+  const auto kernel = small
                           ? (c.dim == 2 ? k_integrate_hash<2, false> : k_integrate_hash<3, false>)
                           : (c.dim == 2 ? k_integrate_hash<2, true> : k_integrate_hash<3, true>);
   SPH_LAUNCH(ws, "integrate_hash", st,
@@ -1604,6 +1626,7 @@ int bin_finish(sph_ws* ws, int bank, const float* r, bool want_pos, const int64_
              k_cell_sort<3><<<cdiv(ws->ncell * 64, 256), 256, 0, st>>>(
                  B.cell_start, ws->unsorted, B.perm, B.iperm, ws->ncell, nullptr, nullptr,
                  Grid{}, ws->cell_count));
+  ws->count_dirty = false;
   if (!want_pos) return SPH_OK;
   if (c.dim == 2)
     SPH_LAUNCH(ws, "gather_pos", st,
@@ -1621,6 +1644,7 @@ int bin_particles(sph_ws* ws, int bank, const float* r, const int64_t* prev_info
   Grid g = make_grid(c);
   if (!bins_small(n, ws->ncell)) {
     const auto kernel = c.dim == 2 ? k_hash_count<2> : k_hash_count<3>;
+    ws->count_dirty = true;
     SPH_LAUNCH(ws, "hash_count", st,
                kernel<<<cdiv(n, kBlock), kBlock, 0, st>>>(
                    r, n, g, ws->cell_count, ws->pcell, ws->pslot, nullptr, info, prev_info));
@@ -1760,6 +1784,7 @@ int skin_begin(sph_ws* ws, const float* r, const float* u, const float* dudt, co
   const Grid g = make_grid(c);
   const Grid gs = skin_grid(ws);
   const unsigned nb = (unsigned)cdiv(n, kBlock);
+  ws->count_dirty = true;
   if (c.dim == 2)
     SPH_LAUNCH(ws, "integrate_skin", st,
                k_integrate_skin<2><<<nb, kBlock, 0, st>>>(
@@ -1777,9 +1802,11 @@ int skin_begin(sph_ws* ws, const float* r, const float* u, const float* dudt, co
       SPH_LAUNCH(ws, "skin_bin", st, (k_bin_small<2, true><<<1, kBinThreads, 0, st>>>(b)));
     else
       SPH_LAUNCH(ws, "skin_bin", st, (k_bin_small<3, true><<<1, kBinThreads, 0, st>>>(b)));
+    ws->count_dirty = false;
     return SPH_OK;
   }
   const int cb = (int)cdiv(ws->ncell, kCellsBlock);
+  S.count_dirty = true;
   if (c.dim == 2)
     SPH_LAUNCH(ws, "skin_hash", st,
                k_skin_hash<2><<<nb + cb, kBlock, 0, st>>>(r_out, n, gs, S.cell_count, ws->pcell,
@@ -1792,6 +1819,7 @@ int skin_begin(sph_ws* ws, const float* r, const float* u, const float* dudt, co
                                                          ws->pslot, S.flag, ws->cell_count,
                                                          ws->ncell, cb, info,
                                                          (int64_t)c.cell_capacity));
+  ws->count_dirty = false;
   const int rc = scan<int32_t>(ws, "skin_scan", S.cell_count, S.ncell, S.b.cell_start,
                                (int32_t*)ws->scan_tmp, nullptr, -1, S.flag, st);
   if (rc) return rc;
@@ -1808,6 +1836,7 @@ int skin_begin(sph_ws* ws, const float* r, const float* u, const float* dudt, co
                k_cell_sort<3><<<cdiv(S.ncell * 64, 256), 256, 0, st>>>(
                    S.b.cell_start, ws->unsorted, S.b.perm, S.b.iperm, S.ncell, S.flag, r_out, gs,
                    S.cell_count));
+  S.count_dirty = false;
   return SPH_OK;
 }
 
@@ -1887,9 +1916,11 @@ int pair_offsets(sph_ws* ws, int bank, hipStream_t st) {
 }
 
 // ------------------------------------------------------------ ensembles
-// Batched forms of the skin-step phases above (skin_begin, skin_build,
-// skin_finish): one launch serves every member.  Per-member arguments are
-// those the single-simulation launches pass; the bodies are shared.
+// Batched forms of the skin-step phases above (skin_begin, skin_build): one
+// launch serves every member.  Per-member arguments are those the
+// single-simulation launches pass; the bodies are shared.  The reductions that
+// ride in a single simulation's sweeps (skin_build_tail, skin_step_tail) are
+// launches of their own here, as is the reference-grid occupancy.
 struct EnsInteg {
   const float *r, *u, *dudt, *dvdt;
   float *r_out, *u_out, *v_out;
@@ -1922,6 +1953,7 @@ struct EnsBin {  // skin-grid binning, all gated on the member's rebuild flag
 
 struct EnsNL {
   int n = 0;
+  std::vector<sph_ws*> ws;
   EnsInteg* integ = nullptr;
   EnsCells* cells = nullptr;
   EnsBin* bin = nullptr;
@@ -2036,6 +2068,7 @@ int ens_nl_create(const std::vector<EnsMember>& members, EnsNL** out) {
   }
   EnsNL* t = new EnsNL;
   t->n = n;
+  for (const EnsMember& m : members) t->ws.push_back(m.ws);
   int rc = upload(integ, &t->integ);
   if (!rc) rc = upload(cells, &t->cells);
   if (!rc) rc = upload(bin, &t->bin);
@@ -2063,6 +2096,7 @@ void ens_nl_destroy(EnsNL* t) {
 
 int ens_skin_begin(EnsNL* t, int dim, const EnsMap& part, const EnsMap& cells, sph_ws* prof,
                    hipStream_t st) {
+  for (sph_ws* ws : t->ws) ws->count_dirty = true;
   if (dim == 2)
     SPH_LAUNCH(prof, "ens_integrate_skin", st,
                k_integrate_skin_ens<2><<<part.blocks, kBlock, 0, st>>>(t->integ, part.d));
@@ -2071,6 +2105,10 @@ int ens_skin_begin(EnsNL* t, int dim, const EnsMap& part, const EnsMap& cells, s
                k_integrate_skin_ens<3><<<part.blocks, kBlock, 0, st>>>(t->integ, part.d));
   SPH_LAUNCH(prof, "ens_cells_max", st,
              k_cells_max_ens<<<t->n, kCellsThreads, 0, st>>>(t->cells));
+  for (sph_ws* ws : t->ws) {
+    ws->count_dirty = false;
+    ws->sk.count_dirty = true;
+  }
   if (dim == 2)
     SPH_LAUNCH(prof, "ens_skin_hash", st,
                k_hash_count_ens<2><<<part.blocks, kBlock, 0, st>>>(t->bin, part.d));
@@ -2086,6 +2124,7 @@ int ens_skin_begin(EnsNL* t, int dim, const EnsMap& part, const EnsMap& cells, s
   else
     SPH_LAUNCH(prof, "ens_skin_sort", st,
                k_cell_sort_ens<3><<<cells.blocks, 256, 0, st>>>(t->bin, cells.d));
+  for (sph_ws* ws : t->ws) ws->sk.count_dirty = false;
   return SPH_OK;
 }
 
@@ -2386,6 +2425,9 @@ extern "C" int sph_nl_build(sph_ws* ws, int bank, const float* r, const int64_t*
   int rc = check_ws(ws, bank);
   if (rc) return rc;
   if (!r || !info) { set_error("sph_nl_build: null"); return SPH_ERR_ARG; }
+  const HistogramGuard guard{ws, st};
+  rc = clean_histograms(ws, st);
+  if (rc) return rc;
   rc = bin_particles(ws, bank, r, prev_info, info, st);
   if (rc) return rc;
   rc = build_pairs(ws, bank, info, st);

@@ -583,6 +583,9 @@ extern "C" int sph_step(sph_ws* ws, int bank, const sph_solver_params* prm, floa
   if (!in->dudt || !in->dvdt) { set_error("sph_step: dudt/dvdt required"); return SPH_ERR_ARG; }
   if (in->g_ext) { set_error("sph_step: position-dependent g_ext is not fused"); return SPH_ERR_ARG; }
   const int n = ws->cfg.n, dim = prm->dim;
+  const HistogramGuard guard{ws, st};
+  rc = clean_histograms(ws, st);
+  if (rc) return rc;
   if (bank == kSkinBank) {
     // 1. kick/drift + rebuild test + reference-grid occupancy; skin binning if needed
     rc = skin_begin(ws, in->r, in->u, in->dudt, in->dvdt, r_out, out->u, out->v, dt, tvf_coef,

@@ -63,7 +63,11 @@ struct sph_ws {
   int32_t ell_overflow = 0;
   int64_t bytes = 0;
   // binning scratch (shared by both banks)
-  int32_t* cell_count = nullptr;  // ncell
+  // The cell histogram: ncell, all zero between builds (the sort, or for skin
+  // lists the hash, clears it).  count_dirty: a launch that adds to it has been
+  // issued and the one that clears it has not (clean_histograms).
+  int32_t* cell_count = nullptr;
+  bool count_dirty = false;
   int32_t* pcell = nullptr;       // N: cell of each original particle
   int32_t* pslot = nullptr;       // N: arrival slot inside the cell
   int32_t* unsorted = nullptr;    // N: ids scattered by arrival order
@@ -89,7 +93,8 @@ struct sph_ws {
     float cell_size[3] = {1.0f, 1.0f, 1.0f};
     int64_t ncell = 0;
     int32_t lane_width = 0;
-    int32_t* cell_count = nullptr;  // ncell, all zero between builds
+    int32_t* cell_count = nullptr;  // ncell, all zero between builds (the sort clears it)
+    bool count_dirty = false;
     int32_t* flag = nullptr;        // device: 1 = rebuild the lists this step
     float4* posb = nullptr;         // N: position of each original id at the last build
     sph::Bank b;                    // perm, iperm, cell_start, pos, ell, cnt of the lists
@@ -128,6 +133,19 @@ int hip_fail(hipError_t e, const char* where);
 // profiling wrappers around a launch
 void prof_begin(sph_ws* ws, const char* name, hipStream_t s);
 void prof_end(sph_ws* ws, hipStream_t s);
+
+// Clears the histograms that an earlier build left with counts in them.  Those
+// of a build that ends early, on a launch that reports an error (also one that
+// a call before it left), would shift the cell starts of the next and place its
+// particles past the end of the sorted arrays.
+int clean_histograms(sph_ws* ws, hipStream_t s);
+// ... as the build's entry point returns, for the replays of graphs captured
+// before; where that fails too, the next call does it.
+struct HistogramGuard {
+  sph_ws* ws;
+  hipStream_t s;
+  ~HistogramGuard();
+};
 }  // namespace sph
 
 #define SPH_CHECK_LAUNCH(where)                                  \

@@ -147,7 +147,7 @@ extern "C" int sph_ws_create(const sph_nl_config* cfg, sph_ws** out) {
   A(ws->eta_varies, 1);
   A(ws->DL0, N); A(ws->DL1, N); A(ws->DL2, N); A(ws->DG0, N); A(ws->DG1, N);
 #undef A
-  // the cell histogram is kept all-zero between launches (scans clear it)
+  // the cell histogram is kept all-zero between builds
   if (rc == SPH_OK) {
     hipError_t e = hipMemset(ws->cell_count, 0, sizeof(int32_t) * (size_t)(ncell ? ncell : 1));
     if (e == hipSuccess) e = hipMemset(ws->eta_varies, 0, sizeof(int32_t));
