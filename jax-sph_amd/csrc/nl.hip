@@ -19,6 +19,7 @@
 #include "sph_device.h"
 #include "sph_internal.h"
 #include "sweep.h"
+#include "tile_band.h"
 
 namespace sph {
 
@@ -820,9 +821,7 @@ struct BuildArgs {
   // rebuild, so rounding at its outer edge cannot drop a pair that matters.)
   float lo, hi;
   int fast;
-  // the matrix-core filter of k_nl_tile: below tlo in, at or above thi out,
-  // in between the filter above decides
-  float tlo, thi;
+  TileBand tile;  // where the filter of k_nl_tile decides, the one above elsewhere
   int range;  // consecutive sorted particles whose pieces a workgroup of k_nl_tile takes
   int n, npad, lane_width, mask_self;
   int64_t* part;          // [2 * gridDim.x]: pairs found and largest list, per workgroup
@@ -1195,9 +1194,10 @@ __device__ __forceinline__ void nl_tile_body(ColdArgs* args, const int blk, cons
       float aa = dist2<DIM>(ax, ay, az);
       // d below is the square less `mid`; hits are under -width, and the
       // exact filter decides within width
-      const float mid = 0.5f * (a->tlo + a->thi);
-      float width = 0.5f * (a->thi - a->tlo);
-      const bool inside = fabsf(ax) <= csx && fabsf(ay) <= csy && (DIM == 2 || fabsf(az) <= csz);
+      const float mid = 0.5f * (a->tile.lo + a->tile.hi);
+      float width = 0.5f * (a->tile.hi - a->tile.lo);
+      const bool inside = fabsf(ax) <= a->tile.inside[0] && fabsf(ay) <= a->tile.inside[1] &&
+                          (DIM == 2 || fabsf(az) <= a->tile.inside[2]);
       ax *= -2.0f;
       ay *= -2.0f;
       az *= -2.0f;
@@ -1652,25 +1652,6 @@ int bin_particles(sph_ws* ws, int bank, const float* r, const int64_t* prev_info
   return bin_finish(ws, bank, r, true, prev_info, info, st);
 }
 
-// The band of k_nl_tile's filter around cutoff_sq: outside it the filter of
-// nl_build_body decides the same.  Per component the exact metric is within
-// 2 ulp(box) of the true one, the fast square within 1 and this one (its
-// centre less an image) within 1: 2 reach sqrt(3) 3 ulp(box) < 16 reach
-// ulp(box).  The expanded square loses at most 15 2^-24 (|a| + |b|)^2, with
-// |a| + |b| <= sqrt(d) cell + reach for a pair at `reach`.
-static void tile_band(BuildArgs& a, float reach, int dim) {
-  double maxbox = 0.0, cell = 0.0;
-  for (int d = 0; d < dim; ++d) {
-    maxbox = std::fmax(maxbox, (double)a.box[d]);
-    cell = std::fmax(cell, (double)a.g.cs[d]);
-  }
-  const double ulp_box = std::nextafter((float)maxbox, INFINITY) - (float)maxbox;
-  const double m = std::sqrt((double)dim) * cell + reach;
-  const double band = 16.0 * reach * ulp_box + 16.0 * std::ldexp(m * m, -23);
-  a.tlo = (float)(a.cutoff_sq - band);
-  a.thi = (float)(a.cutoff_sq + band);
-}
-
 // The cell-adjacent image is the minimum image of every pair within the cutoff
 // when each side has >= 5 cells (2 cells < box/2).  Both the fast and the exact
 // squared distance are then within a few ulp(box) per component of the true
@@ -1731,7 +1712,7 @@ int build_pairs(sph_ws* ws, int bank, int64_t* info, hipStream_t st) {
   a.fast = fast_filter(c);
   a.range = tile_range(c.dim, c.n);
   cut_band(c, &a.lo, &a.hi);
-  tile_band(a, c.cutoff, c.dim);
+  a.tile = tile_band(a.box, a.g.cs, c.dim, c.cutoff, a.cutoff_sq);
   constexpr int T2 = tpp_of(2), T3 = tpp_of(3);
   const bool d2 = c.dim == 2;
   const auto kernel = tiled(c)    ? (d2 ? k_nl_tile<2, T2> : k_nl_tile<3, T3>)
@@ -1864,7 +1845,7 @@ static BuildArgs skin_build_args(sph_ws* ws, int64_t* info) {
   a.fast = 1;
   a.range = tile_range(c.dim, c.n);
   a.lo = a.hi = S.reach_sq;
-  tile_band(a, c.cutoff + S.skin, c.dim);
+  a.tile = tile_band(a.box, a.g.cs, c.dim, c.cutoff + S.skin, a.cutoff_sq);
   a.n = c.n;
   a.npad = ws->npad;
   a.lane_width = S.lane_width;
