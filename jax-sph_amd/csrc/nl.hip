@@ -816,9 +816,7 @@ struct BuildArgs {
   // fast filter: squared distances of the cell-adjacent image below `lo` are
   // in, above `hi` out; the band [lo, hi) bounds the difference between that
   // and the exact reference metric, and is decided by the exact predicate.
-  // (Skin lists: lo = hi, no band.  A skin list must hold every pair within
-  // cutoff + 0.98 skin, the most two particles can close before the next
-  // rebuild, so rounding at its outer edge cannot drop a pair that matters.)
+  // (Skin lists: lo = hi, no band; see test_range.)
   float lo, hi;
   int fast;
   TileBand tile;  // where the filter of k_nl_tile decides, the one above elsewhere
@@ -847,7 +845,14 @@ struct BuildArgs {
 // build's registers allow.
 constexpr int kStage = 24;
 
-template <int DIM, int TPP, bool ORDERED>
+// BAND = false (skin lists): pairs are kept by the fast squared distance
+// alone.  A skin list must hold every pair within cutoff + 0.98 skin (the
+// most two particles can close before the next rebuild), so rounding at its
+// outer edge, cutoff + skin, cannot drop a pair that matters.  Skin lists of
+// 160,000 and 409,600 2D particles 30.6 and 52.6 us, with the band's
+// comparisons and each candidate's index clamped 37.3 and 62.1; of an ensemble
+// of 64 members (565,000 2D particles) 129 and 157.
+template <int DIM, int TPP, bool ORDERED, bool BAND>
 __device__ __forceinline__ void test_range(const BuildArgs& a, int s, int h, const float4 ps,
                                            int sid, int lo, int hi, const float* img,
                                            int32_t* __restrict__ out0, int32_t* stage0,
@@ -863,15 +868,31 @@ __device__ __forceinline__ void test_range(const BuildArgs& a, int s, int h, con
     unsigned mask = 0u;
     for (int t0 = 0; t0 < nb; t0 += G) {
       float4 pg[G];
+      if (BAND) {
 #pragma unroll
-      for (int u = 0; u < G; ++u) {
-        const int b = c0 + (t0 + u) * TPP;
-        const int bc = b < hi ? b : hi - 1;
-        __builtin_assume(bc >= 0);  // sorted slots: no sign extension in the address
-        pg[u] = a.pos[bc];
+        for (int u = 0; u < G; ++u) {
+          const int b = c0 + (t0 + u) * TPP;
+          const int bc = b < hi ? b : hi - 1;
+          __builtin_assume(bc >= 0);  // sorted slots: no sign extension in the address
+          pg[u] = a.pos[bc];
+        }
+      } else {
+        // skin builds read past the range into the padded tail (kSkinPosPad),
+        // from one address with constant offsets; those candidates are masked
+        // off below
+        __builtin_assume(c0 >= 0);
+        const float4* __restrict__ pb = a.pos + (c0 + t0 * TPP);
+#pragma unroll
+        for (int u = 0; u < G; ++u) pg[u] = pb[u * TPP];
       }
       unsigned got = 0u;  // bit u: candidate t0 + u is a pair
-      if (a.fast) {
+      if (!BAND) {
+#pragma unroll
+        for (int u = 0; u < G; ++u) {
+          const float4 pb = pg[u];
+          got |= dist2<DIM>(sx - pb.x, sy - pb.y, sz - pb.z) < a.lo ? 1u << u : 0u;
+        }
+      } else if (a.fast) {
         bool near = false;  // some candidate lies in the band around the cutoff
 #pragma unroll
         for (int u = 0; u < G; ++u) {
@@ -979,7 +1000,7 @@ __device__ __forceinline__ void store_count(const Args& a, int s, int h, int sha
 // the receivers with d^2 < cutoff^2 and stores them in its own sub-list.
 // blk: the workgroup's block within this list's grid; it also indexes the
 // workgroup's partials.
-template <int DIM, int TPP, bool ORDERED>
+template <int DIM, int TPP, bool ORDERED, bool BAND>
 __device__ __forceinline__ void nl_build_body(const BuildArgs& a, const int blk) {
   __shared__ int32_t stage_buf[kStage][kBlock];
   if (a.gate && *a.gate == 0) return;  // uniform over the list's grid
@@ -993,7 +1014,7 @@ __device__ __forceinline__ void nl_build_body(const BuildArgs& a, const int blk)
     int32_t* stage = &stage_buf[0][threadIdx.x - h];    // stage column of lane 0 of s
     float img[3] = {0.0f, 0.0f, 0.0f};
     if (!a.g.use_cells) {
-      test_range<DIM, TPP, ORDERED>(a, s, h, ps, sid, 0, a.n, img, out, stage, count);
+      test_range<DIM, TPP, ORDERED, BAND>(a, s, h, ps, sid, 0, a.n, img, out, stage, count);
     } else {
       int c[3];
       cell_coords<DIM>(ps, a.g, c);
@@ -1013,7 +1034,7 @@ __device__ __forceinline__ void nl_build_body(const BuildArgs& a, const int blk)
           const int row = (cz * ny + cy) * nx;
           if (c[0] >= 1 && c[0] + 1 < nx) {
             img[0] = 0.0f;
-            test_range<DIM, TPP, ORDERED>(a, s, h, ps, sid, a.cell_start[row + c[0] - 1],
+            test_range<DIM, TPP, ORDERED, BAND>(a, s, h, ps, sid, a.cell_start[row + c[0] - 1],
                                     a.cell_start[row + c[0] + 2], img, out, stage, count);
           } else {
             for (int dx = -1; dx <= 1; ++dx) {
@@ -1021,7 +1042,7 @@ __device__ __forceinline__ void nl_build_body(const BuildArgs& a, const int blk)
               img[0] = 0.0f;
               if (cx < 0) { cx += nx; img[0] = -a.box[0]; }
               else if (cx >= nx) { cx -= nx; img[0] = a.box[0]; }
-              test_range<DIM, TPP, ORDERED>(a, s, h, ps, sid, a.cell_start[row + cx],
+              test_range<DIM, TPP, ORDERED, BAND>(a, s, h, ps, sid, a.cell_start[row + cx],
                                       a.cell_start[row + cx + 1], img, out, stage, count);
             }
           }
@@ -1044,9 +1065,9 @@ __device__ __forceinline__ void nl_build_body(const BuildArgs& a, const int blk)
   build_partials(a.part, blk, share, count);
 }
 
-template <int DIM, int TPP, bool ORDERED>
+template <int DIM, int TPP, bool ORDERED, bool BAND>
 __global__ __launch_bounds__(kBlock, ORDERED ? 1 : 6) void k_nl_build(BuildArgs a) {
-  nl_build_body<DIM, TPP, ORDERED>(a, logical_block(a.remap));
+  nl_build_body<DIM, TPP, ORDERED, BAND>(a, logical_block(a.remap));
 }
 
 // ------------------------------------------------- pair build, matrix cores
@@ -1715,9 +1736,10 @@ int build_pairs(sph_ws* ws, int bank, int64_t* info, hipStream_t st) {
   a.tile = tile_band(a.box, a.g.cs, c.dim, c.cutoff, a.cutoff_sq);
   constexpr int T2 = tpp_of(2), T3 = tpp_of(3);
   const bool d2 = c.dim == 2;
-  const auto kernel = tiled(c)    ? (d2 ? k_nl_tile<2, T2> : k_nl_tile<3, T3>)
-                      : c.ordered ? (d2 ? k_nl_build<2, T2, true> : k_nl_build<3, T3, true>)
-                                  : (d2 ? k_nl_build<2, T2, false> : k_nl_build<3, T3, false>);
+  const auto kernel =
+      tiled(c)    ? (d2 ? k_nl_tile<2, T2> : k_nl_tile<3, T3>)
+      : c.ordered ? (d2 ? k_nl_build<2, T2, true, true> : k_nl_build<3, T3, true, true>)
+                  : (d2 ? k_nl_build<2, T2, false, true> : k_nl_build<3, T3, false, true>);
   SPH_LAUNCH(ws, "nl_build", st, (kernel<<<build_grid(ws, tiled(c)), kBlock, 0, st>>>(a)));
   return SPH_OK;
 }
@@ -1865,7 +1887,7 @@ int skin_build(sph_ws* ws, int64_t* info, hipStream_t st) {
   const bool tile = skin_tiled(c);
   const auto kernel = c.dim == 3 ? k_nl_tile<3, T3>
                       : tile     ? k_nl_tile<2, T2>
-                                 : k_nl_build<2, T2, false>;
+                                 : k_nl_build<2, T2, false, false>;
   SPH_LAUNCH(ws, "skin_build", st, (kernel<<<build_grid(ws, tile), kBlock, 0, st>>>(a)));
   return SPH_OK;
 }
@@ -2003,7 +2025,7 @@ __global__ __launch_bounds__(kBlock, 6) void k_nl_build_ens(const BuildArgs* __r
   if constexpr (DIM == 3)
     nl_tile_body<DIM, TPP>((ColdArgs*)(t + m.sim), m.blk, kBlock / TPP);
   else
-    nl_build_body<DIM, TPP, false>(t[m.sim], m.blk);
+    nl_build_body<DIM, TPP, false, false>(t[m.sim], m.blk);
 }
 
 // one workgroup per member

@@ -29,6 +29,11 @@ struct Bank {
 // scheduler enough independent gathers to hide memory latency.
 __host__ __device__ constexpr int tpp_of(int dim) { return dim == 3 ? 4 : 2; }
 
+// Spare entries after the skin lists' sorted build positions: the lanes' skin
+// build reads each batch of candidates from one address with constant offsets,
+// up to 31 TPP entries past a cell range, without clamping each one.
+constexpr int kSkinPosPad = 128;
+
 // Consecutive sorted particles of a workgroup of the matrix-core pair build,
 // whose four wavefronts take in turn the pieces (up to 12 or 16 particles of
 // one cell) that start there.  A workgroup lasts as long as the wavefront with

@@ -210,7 +210,7 @@ extern "C" int sph_skin_enable(sph_ws* ws, float skin, int32_t width) {
   A(S.b.cell_start, ncell + 1);
   A(S.b.ell, ws->tpp * lw * npad);
   A(S.b.cnt, ws->tpp * npad);
-  A(S.b.pos, N);
+  A(S.b.pos, N + kSkinPosPad);  // last, so that its padding moves no other buffer
 #undef A
   if (rc == SPH_OK) {
     const int32_t one = 1;  // the first step builds the lists

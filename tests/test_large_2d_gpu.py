@@ -1,0 +1,50 @@
+"""2D sets beyond 150,000 particles, whose builds compare candidate by candidate:
+the exact list of a lattice with pairs exactly at the cutoff, and the skin list
+of a few steps, against the oracle's per-step search."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import nl_oracle as nlo
+
+pytestmark = pytest.mark.gpu
+
+js = pytest.importorskip("jax_sph_amd")
+from jax_sph_amd import partition  # noqa: E402
+from jax_sph_amd.jax_md import space  # noqa: E402
+from tests.test_step_gpu import _make  # noqa: E402
+
+
+@pytest.mark.parametrize("mask_self", [True, False])
+def test_lattice_pairs_at_the_cutoff(mask_self):
+    side = 388
+    x = (np.arange(side) + 0.5) / side
+    r = np.stack(np.meshgrid(x, x, indexing="ij"), -1).reshape(-1, 2).astype(np.float32)
+    n = len(r)
+    disp, _ = space.periodic(side=np.ones(2))
+    fn = partition.neighbor_list(disp, np.ones(2), r_cutoff=3 / side, mask_self=mask_self,
+                                 format=partition.Sparse)
+    nb = fn.allocate(torch.tensor(r, device="cuda"))
+    want = nlo.sorted_pairs(nlo.NeighborSearch(np.ones(2), 3 / side,
+                                               mask_self=mask_self).allocate(r).idx, n)
+    assert np.array_equal(nlo.sorted_pairs(nb.idx.cpu().numpy(), n), want)
+
+
+def test_skin_list():
+    cfg, state, nb, adv, R, fn, *_ = _make("tgv", {"case": {"dim": 2, "dx": 1 / 400,
+                                                             "r0_noise_factor": 0.1}})
+    assert nb.workspace.skin_on and nb.workspace.n == 160000
+    ref_nb = R.ns.allocate(state["r"].cpu().numpy())
+    st = state
+    for k in range(3):
+        if k == 2:
+            nb.workspace.tune("skin_rebuild", 1)
+        st, nb = adv(cfg.solver.dt, st, nb)
+        r = st["r"].cpu().numpy()
+        ref_nb = R.ns.update(r, ref_nb)
+        want = nlo.sorted_pairs(ref_nb.idx, len(r))
+        assert np.array_equal(nlo.sorted_pairs(nb.idx.cpu().numpy(), len(r)), want), k
+        info = nb.info.cpu().numpy()
+        assert int(info[0]) == int(ref_nb.error) and int(info[1]) == ref_nb.occupancy
+        assert int(info[3]) == np.bincount(want[1], minlength=len(r)).max()
+        assert (int(info[7]) > 0) == (k != 1)   # the steps that rebuilt
