@@ -133,7 +133,10 @@ int64_t sph_ws_bytes(const sph_ws *ws);
  * sph_skin_enable (synchronous; outside graph capture).
  * "ell_overflow" (1): for a workspace whose ell_width is below 3^dim x
  * cell_capacity, a particle with more pairs than fit raises
- * SPH_NEIGHBOR_LIST_OVERFLOW (default 0: such a width is not expected). */
+ * SPH_NEIGHBOR_LIST_OVERFLOW (default 0: such a width is not expected).
+ * "occupied_cells" (default 0, not known): cells of the grid that hold
+ * particles, by which the faster of two pair builds is chosen; the lists are
+ * the same. */
 int sph_ws_tune(sph_ws *ws, const char *key, int64_t value);
 
 /* ---- neighbour search: jax_sph/partition.py:492-571 + jax_md/partition.py:723-1026 */

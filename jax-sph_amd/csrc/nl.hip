@@ -1086,8 +1086,8 @@ __global__ __launch_bounds__(kBlock, ORDERED ? 1 : 6) void k_nl_build(BuildArgs 
 // Bound by the issue of instructions (vector 61%, scalar 64% of the cycles), 10
 // for a particle and 64 candidates; a lane that tests candidates of its own
 // takes 9 per candidate and 25 per hit, in a loop as long as the wavefront's
-// longest.  Exact list of 1,000,000 3D particles 647 -> 421 us; tiled() has the
-// other sizes.
+// longest.  Exact list of 1,000,000 3D particles 647 -> 421 us; tile_pays() has
+// the other sizes.
 // A stage entry is 16 bits (segment and offset in it, from which the sorted
 // index follows), so that 7 workgroups' stages fit a CU's LDS; entries past
 // the stage, and those of segments over 2,047 long, go straight to the buffer.
@@ -1684,18 +1684,56 @@ static bool fast_filter(const sph_nl_config& c) {
   return true;
 }
 
-// Which lists k_nl_tile builds: its filter is the fast one's, and ordered (half)
-// lists compare ids candidate by candidate.  In 2D its 64 candidates at a time
-// are two chunks half full for each 9 particles, which pays while SIMDs are
-// idle anyway; microseconds by k_nl_build and so (exact lists):
-//   2D 900 particles 25.2, 9.6; 10,000 24.4, 12.3; 40,000 26.0, 14.1;
-//   160,000 33.3, 33.9; 810,000 90, 130
-//   3D 8,000 84.9, 30.8; 64,000 97.1, 55.4; 262,144 221.6, 127.9;
-//   1,000,000 647, 421; Wendland C2 (18 a cell) 91,125 72.0, 36.1
-static bool tiled(const sph_nl_config& c) {
-  return fast_filter(c) && !c.ordered && (c.dim == 3 || c.n < 150000);
+// Where k_nl_tile is the faster build, by the particles an occupied cell holds
+// and the pairs a particle has (both means).  A wavefront spends a piece's time
+// on however few particles the piece has, so cells must hold some; and hits
+// past a particle's stage cost its slow path, so most lists must fit.  Small
+// sets leave SIMDs idle, where both matter less.  In 2D a piece's 64 candidates
+// at a time are two chunks half full for each 9 particles, which pays until
+// there are pieces for every SIMD: `most` occupied cells.
+// Microseconds by the lanes' build and so, noisy lattices, exact lists:
+//   3D 9,000 particles, 1 a cell 44, 34; 30,000, 1.4 a cell 37, 38; 2.1 38, 30;
+//   59 (245 pairs) 137, 124
+//   60,000, 1.3 a cell 43, 59; 3.2 48, 38; 28 93, 53; 45 (189 pairs) 144, 164
+//   300,000, 2.6 a cell 139, 142; 4.1 136, 101; 38 (157 pairs) 323, 184;
+//   51 (216 pairs) 411, 496
+//   2D 20,000, 2 a cell 18, 20; 3 19, 17; 32 (100 pairs) 56, 32
+//   60,000, 3 a cell 21, 25; 9 27, 20; 12 (37 pairs) 31, 23; 16 (51 pairs, 3,720
+//   cells) 38, 44; 20 (3,030 cells) 46, 35
+//   145,000, 4 a cell 25, 36; 9 (16,100 cells) 33, 33
+static bool tile_pays(int dim, int64_t n, double occupied, const float* cell, float reach,
+                      double most) {
+  const double held = (double)n / occupied;
+  double pairs = held * (dim == 3 ? 4.19 : 3.14);
+  for (int d = 0; d < dim; ++d) pairs *= (double)reach / (double)cell[d];
+  if (dim == 3)
+    return held >= (n < 15000 ? 1.0 : n < 40000 ? 1.5 : 3.0) && pairs <= (n < 40000 ? 300.0 : 158.0);
+  return held >= 2.5 && occupied <= most && (pairs <= 43.0 || occupied <= 3200.0);
 }
-static bool skin_tiled(const sph_nl_config& c) { return c.dim == 3 || c.n < 150000; }
+
+// Cells of the reference grid that hold particles: as told (sph_ws_tune), else
+// as if the particles were spread over all of them.
+static double occupied_cells(const sph_ws* ws) {
+  if (ws->occupied > 0) return (double)ws->occupied;
+  return (double)(ws->ncell < ws->cfg.n ? ws->ncell : (int64_t)ws->cfg.n);
+}
+
+// Exact lists: k_nl_tile's filter is the fast one's, and ordered (half) lists
+// compare ids candidate by candidate.
+static bool tiled(const sph_ws* ws) {
+  const auto& c = ws->cfg;
+  return fast_filter(c) && !c.ordered &&
+         tile_pays(c.dim, c.n, occupied_cells(ws), c.cell_size, c.cutoff, 15000.0);
+}
+// Skin lists, which the lanes build without a band: 2D 48,400 particles 22.7 and
+// 20.2 us, 67,600 (6,400 cells) 24.5 and 23.9, 78,400 (7,400) 25.3 and 26.1,
+// 136,900 30.7 and 33.2; Wendland C2 14,400 16.1 and 12.2, 57,600 17.2 and 19.9.
+static bool skin_tiled(const sph_ws* ws) {
+  const auto& c = ws->cfg;
+  const auto& S = ws->sk;
+  const double occupied = occupied_cells(ws) * (double)S.ncell / (double)ws->ncell;
+  return tile_pays(c.dim, c.n, occupied, S.cell_size, c.cutoff + S.skin, 7000.0);
+}
 
 static unsigned build_grid(const sph_ws* ws, bool tile) {
   const auto& c = ws->cfg;
@@ -1735,19 +1773,19 @@ int build_pairs(sph_ws* ws, int bank, int64_t* info, hipStream_t st) {
   cut_band(c, &a.lo, &a.hi);
   a.tile = tile_band(a.box, a.g.cs, c.dim, c.cutoff, a.cutoff_sq);
   constexpr int T2 = tpp_of(2), T3 = tpp_of(3);
-  const bool d2 = c.dim == 2;
+  const bool d2 = c.dim == 2, tile = tiled(ws);
   const auto kernel =
-      tiled(c)    ? (d2 ? k_nl_tile<2, T2> : k_nl_tile<3, T3>)
+      tile        ? (d2 ? k_nl_tile<2, T2> : k_nl_tile<3, T3>)
       : c.ordered ? (d2 ? k_nl_build<2, T2, true, true> : k_nl_build<3, T3, true, true>)
                   : (d2 ? k_nl_build<2, T2, false, true> : k_nl_build<3, T3, false, true>);
-  SPH_LAUNCH(ws, "nl_build", st, (kernel<<<build_grid(ws, tiled(c)), kBlock, 0, st>>>(a)));
+  SPH_LAUNCH(ws, "nl_build", st, (kernel<<<build_grid(ws, tile), kBlock, 0, st>>>(a)));
   return SPH_OK;
 }
 
 // What an exact build leaves to reduce: occupancy info[1], largest list
 // info[3], and the overflow bit when max_occupancy >= 0.
 Reduce build_tail(sph_ws* ws, int64_t max_occupancy, int64_t* info) {
-  const int blocks = (int)build_grid(ws, tiled(ws->cfg));
+  const int blocks = (int)build_grid(ws, tiled(ws));
   return Reduce{ws->part_build, blocks, &info[1], &info[3], info, max_occupancy, nullptr, nullptr};
 }
 
@@ -1884,10 +1922,9 @@ int skin_build(sph_ws* ws, int64_t* info, hipStream_t st) {
   auto& S = ws->sk;
   const BuildArgs a = skin_build_args(ws, info);
   constexpr int T2 = tpp_of(2), T3 = tpp_of(3);
-  const bool tile = skin_tiled(c);
-  const auto kernel = c.dim == 3 ? k_nl_tile<3, T3>
-                      : tile     ? k_nl_tile<2, T2>
-                                 : k_nl_build<2, T2, false, false>;
+  const bool d2 = c.dim == 2, tile = skin_tiled(ws);
+  const auto kernel = tile ? (d2 ? k_nl_tile<2, T2> : k_nl_tile<3, T3>)
+                           : (d2 ? k_nl_build<2, T2, false, false> : k_nl_build<3, T3, false, false>);
   SPH_LAUNCH(ws, "skin_build", st, (kernel<<<build_grid(ws, tile), kBlock, 0, st>>>(a)));
   return SPH_OK;
 }
@@ -1895,7 +1932,7 @@ int skin_build(sph_ws* ws, int64_t* info, hipStream_t st) {
 // What a skin build leaves to reduce: the largest list of one particle ->
 // info[7] (only on a rebuild).
 Reduce skin_build_tail(sph_ws* ws, int64_t* info) {
-  const int blocks = (int)build_grid(ws, skin_tiled(ws->cfg));
+  const int blocks = (int)build_grid(ws, skin_tiled(ws));
   return Reduce{ws->part_build, blocks, nullptr, &info[7], info, -1, ws->sk.flag, nullptr};
 }
 
@@ -2015,7 +2052,7 @@ __global__ __launch_bounds__(256) void k_cell_sort_ens(const EnsBin* __restrict_
 }
 
 // The members of a 2D ensemble are many particles together, where the lanes'
-// build is the faster one (see tiled()).
+// build is the faster one (see skin_tiled()).
 template <int DIM, int TPP>
 __global__ __launch_bounds__(kBlock, 6) void k_nl_build_ens(const BuildArgs* __restrict__ t,
                                                             const EnsBlock* __restrict__ map) {

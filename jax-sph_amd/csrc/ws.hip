@@ -282,6 +282,11 @@ extern "C" int sph_ws_tune(sph_ws* ws, const char* key, int64_t value) {
     ws->ell_overflow = value ? 1 : 0;
     return SPH_OK;
   }
+  if (std::strcmp(key, "occupied_cells") == 0) {
+    if (value < 0) { set_error("sph_ws_tune: occupied_cells must be >= 0"); return SPH_ERR_ARG; }
+    ws->occupied = value;
+    return SPH_OK;
+  }
   if (std::strcmp(key, "skin_rebuild") == 0) {
     // the next fused step rebuilds the skin lists, as the first step after
     // sph_skin_enable does (synchronous; not for use under graph capture)

@@ -1,0 +1,54 @@
+"""The two pair builds give the same list, entry by entry, wherever the choice
+between them falls: sparse and dense cells, few and many particles, a box that is
+mostly empty, exact and skin lists."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+js = pytest.importorskip("jax_sph_amd")
+from jax_sph_amd import partition  # noqa: E402
+from jax_sph_amd.jax_md import space  # noqa: E402
+from tests.test_step_gpu import _make  # noqa: E402
+
+# particles, cells a side, part of the box that holds them
+SETS = [(2, 3000, 80, 1.0), (2, 3000, 40, 1.0), (2, 3000, 12, 1.0), (2, 3000, 60, 0.3),
+        (2, 45000, 140, 1.0), (2, 45000, 70, 1.0), (2, 45000, 50, 1.0),
+        (3, 5000, 24, 1.0), (3, 5000, 14, 1.0), (3, 5000, 5, 1.0), (3, 5000, 20, 0.4),
+        (3, 41000, 30, 1.0), (3, 41000, 12, 1.0), (3, 41000, 9, 1.0)]
+
+
+@pytest.mark.parametrize("dim,n,cells,part", SETS)
+def test_exact_lists(dim, n, cells, part):
+    r = np.random.default_rng(n + cells).random((n, dim)).astype(np.float32)
+    r[:, 0] *= np.float32(part)
+    cutoff = 0.9995 / cells
+    disp, _ = space.periodic(side=np.ones(dim))
+    fn = partition.neighbor_list(disp, np.ones(dim), r_cutoff=cutoff, format=partition.Sparse)
+    t = torch.tensor(r, device="cuda")
+    nb = fn.allocate(t)
+    idx, info = nb.idx, nb.info
+    assert not bool(nb.did_buffer_overflow)
+    # as if the particles were alone in their cells, and as if ten (in 2D five) shared one
+    for told in (2 * n, n // (10 if dim == 3 else 5), 0):
+        nb.workspace.tune("occupied_cells", told)
+        nb = nb.update(t)
+        assert torch.equal(nb.info[:4], info[:4])
+        assert torch.equal(nb.idx, idx), told
+
+
+@pytest.mark.parametrize("dim,side", [(2, 80), (3, 16), (3, 13), (3, 11)])
+def test_skin_lists(dim, side):
+    """The last two have skin grids of four and three cells a side."""
+    out = []
+    for told in (1 << 30, side ** dim // (20 if dim == 3 else 5)):
+        dx = 2 * np.pi / side if dim == 3 else 1 / side
+        cfg, state, nb, adv, *_ = _make("tgv", {"case": {"dim": dim, "dx": dx,
+                                                         "r0_noise_factor": 0.1}})
+        assert nb.workspace.skin_on
+        nb.workspace.tune("occupied_cells", told)
+        st, nb = adv(cfg.solver.dt, state, nb)
+        out.append((nb.idx, nb.info[:4], st["r"], st["dudt"], st["rho"]))
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
