@@ -2429,8 +2429,10 @@ extern "C" int sph_cell_list(int32_t dim, int32_t n, const float* r, const float
   }
   // cell starts, the largest occupancy into info[2], CELL_LIST_OVERFLOW into info[0]
   SPH_LAUNCH(ws, "fill", st, k_fill<int64_t><<<1, 64, 0, st>>>(info + 2, 1, 0));
-  const int rc = scan<int32_t>(ws, "scan_cells", counts, nc, start, nullptr, info, capacity,
-                               nullptr, st);
+  // (chunk sums in the sorted ids' place, which nothing has written yet)
+  int32_t* const sums = 3 * (int64_t)n >= kScanSums ? unsorted : nullptr;
+  const int rc = scan<int32_t>(ws, "scan_cells", counts, nc, start, sums, info, capacity, nullptr,
+                               st);
   if (rc) return rc;
   if (n == 0) return SPH_OK;
   SPH_LAUNCH(ws, "scatter", st,
