@@ -1244,37 +1244,32 @@ __device__ __forceinline__ void nl_tile_body(ColdArgs* args, const int blk, cons
       int seg = 0;  // the last segment that starts before the candidates seen end
       const int full = (int)row0 + room;
       int tops = (int)row0;  // lane q: the next entry of row q, less q kRow
-      // Candidates are requested kDepth chunks before their tests (past the end:
-      // s0 again): a chunk's tests take less than a load that misses the L2.
-      constexpr int kDepth = 1;
-      unsigned codes[kDepth + 1];  // candidate c0 + 64 k + lane: segment and offset in it
-      // and its position, three words of it: a fourth that nothing reads would
-      // be some other value's register next, which then waits for the load
+      // A chunk of candidates is requested before the tests of the one before
+      // (past the end: s0 again); more ahead gained nothing.
+      // c, at: candidate c0 + lane, its segment and offset in it, and its
+      // position, three words of it: a fourth that nothing reads would be some
+      // other value's register next, which then waits for the load
       struct Xyz { float x, y, z; };
-      Xyz at[kDepth + 1];
-#pragma unroll
-      for (int k = 0; k <= kDepth; ++k) {
-        codes[k] = 0;
-        at[k] = Xyz{0.f, 0.f, 0.f};
-      }
-      for (int c0 = -64 * kDepth; c0 < total; c0 += 64) {
-        const int first_new = c0 + 64 * kDepth;
-        const int o = first_new + lane;
+      unsigned c_next = 0;
+      Xyz at_next{0.f, 0.f, 0.f};
+      for (int c0 = -64; c0 < total; c0 += 64) {
+        const unsigned c = c_next;
+        const Xyz at = at_next;
+        const int o = c0 + 64 + lane;
         int to_j = lane_i(shift, seg);
         unsigned to_c = (unsigned)lane_i((int)code, seg);
         while (seg + 1 < nseg) {
           const int first = lane_i(pre, seg + 1);
-          if (first >= first_new + 64) break;
+          if (first >= c0 + 128) break;
           ++seg;
           const bool on = o >= first;
           const int tj = lane_i(shift, seg), tc = lane_i((int)code, seg);
           to_j = on ? tj : to_j;
           to_c = on ? (unsigned)tc : to_c;
         }
-        at[kDepth] = *(const Xyz*)(pos + (unsigned)(o < total ? o + to_j : s0));
-        codes[kDepth] = (unsigned)o + to_c;
-        const unsigned c = codes[0];
-        const float4 pb = make_float4(at[0].x, at[0].y, at[0].z, 0.0f);
+        at_next = *(const Xyz*)(pos + (unsigned)(o < total ? o + to_j : s0));
+        c_next = (unsigned)o + to_c;
+        const float4 pb = make_float4(at.x, at.y, at.z, 0.0f);
         if (c0 >= 0) {
           const bool valid = c0 + lane < total;
           float cix = 0.0f, ciy = 0.0f, ciz = 0.0f;  // its image
@@ -1369,11 +1364,6 @@ __device__ __forceinline__ void nl_tile_body(ColdArgs* args, const int blk, cons
               tops = lane == q ? t + (int)__popcll(mq) : tops;
             }
           }
-        }
-#pragma unroll
-        for (int k = 0; k < kDepth; ++k) {
-          codes[k] = codes[k + 1];
-          at[k] = at[k + 1];
         }
       }
       // ---- counts, and the staged entries in the order of the buffer's rows
