@@ -134,9 +134,8 @@ int64_t sph_ws_bytes(const sph_ws *ws);
  * "ell_overflow" (1): for a workspace whose ell_width is below 3^dim x
  * cell_capacity, a particle with more pairs than fit raises
  * SPH_NEIGHBOR_LIST_OVERFLOW (default 0: such a width is not expected).
- * "occupied_cells" (default 0, not known): cells of the grid that hold
- * particles, by which the faster of two pair builds is chosen; the lists are
- * the same. */
+ * "pairs" (default 0, not known): about the pairs a list holds (info[1] of one),
+ * by which the faster of two pair builds is chosen; the lists are the same. */
 int sph_ws_tune(sph_ws *ws, const char *key, int64_t value);
 
 /* ---- neighbour search: jax_sph/partition.py:492-571 + jax_md/partition.py:723-1026 */

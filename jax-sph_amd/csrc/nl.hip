@@ -1685,38 +1685,43 @@ static bool fast_filter(const sph_nl_config& c) {
   return true;
 }
 
-// Where k_nl_tile is the faster build, by the particles an occupied cell holds
-// and the pairs a particle has (both means).  A wavefront spends a piece's time
-// on however few particles the piece has, so cells must hold some; and hits
-// past a particle's stage cost its slow path, so most lists must fit.  Small
-// sets leave SIMDs idle, where both matter less.  In 2D a piece's 64 candidates
-// at a time are two chunks half full for each 9 particles, which pays until
-// there are pieces for every SIMD: `most` occupied cells.
+// Where k_nl_tile is the faster build, by the pairs a particle has within reach
+// and the particles that a cell then holds (means over the particles).  A
+// wavefront spends a piece's time on however few particles the piece has, so
+// cells must hold some; and hits past a particle's stage cost its slow path, so
+// most lists must fit.  Small sets leave SIMDs idle, where both matter less.  In
+// 2D a piece's 64 candidates at a time are two chunks half full for each 9
+// particles, which pays until there are pieces for every SIMD: `most` cells.
 // Microseconds by the lanes' build and so, noisy lattices, exact lists:
-//   3D 9,000 particles, 1 a cell 44, 34; 30,000, 1.4 a cell 37, 38; 2.1 38, 30;
-//   59 (245 pairs) 137, 124
-//   60,000, 1.3 a cell 43, 59; 3.2 48, 38; 28 93, 53; 45 (189 pairs) 144, 164
+//   3D 256 particles, 0.3 a cell 39, 30; 9,000, 1 a cell 44, 34; 30,000, 1 a cell
+//   37, 38; 1.9 38, 30; 59 (245 pairs) 137, 124
+//   60,000, 1 a cell 43, 59; 3 48, 38; 27 93, 53; 45 (189 pairs) 144, 164
 //   300,000, 2.6 a cell 139, 142; 4.1 136, 101; 38 (157 pairs) 323, 184;
 //   51 (216 pairs) 411, 496
 //   2D 20,000, 2 a cell 18, 20; 3 19, 17; 32 (100 pairs) 56, 32
 //   60,000, 3 a cell 21, 25; 9 27, 20; 12 (37 pairs) 31, 23; 16 (51 pairs, 3,720
 //   cells) 38, 44; 20 (3,030 cells) 46, 35
 //   145,000, 4 a cell 25, 36; 9 (16,100 cells) 33, 33
-static bool tile_pays(int dim, int64_t n, double occupied, const float* cell, float reach,
+// 5,000 particles, half of them in one 3D cell (650 pairs) 175, 273.
+static constexpr double kBall[] = {0.0, 2.0, 3.14, 4.19};
+static bool tile_pays(int dim, int64_t n, double pairs, const float* cell, float reach,
                       double most) {
-  const double held = (double)n / occupied;
-  double pairs = held * (dim == 3 ? 4.19 : 3.14);
-  for (int d = 0; d < dim; ++d) pairs *= (double)reach / (double)cell[d];
+  double held = pairs / kBall[dim];
+  for (int d = 0; d < dim; ++d) held *= (double)cell[d] / (double)reach;
   if (dim == 3)
-    return held >= (n < 15000 ? 1.0 : n < 40000 ? 1.5 : 3.0) && pairs <= (n < 40000 ? 300.0 : 158.0);
-  return held >= 2.5 && occupied <= most && (pairs <= 43.0 || occupied <= 3200.0);
+    return held >= (n < 15000 ? 0.2 : n < 40000 ? 0.8 : 2.8) && pairs <= (n < 40000 ? 300.0 : 158.0);
+  const double cells = (double)n / held;
+  return held >= 2.5 && cells <= most && (pairs <= 43.0 || cells <= 3200.0);
 }
 
-// Cells of the reference grid that hold particles: as told (sph_ws_tune), else
-// as if the particles were spread over all of them.
-static double occupied_cells(const sph_ws* ws) {
-  if (ws->occupied > 0) return (double)ws->occupied;
-  return (double)(ws->ncell < ws->cfg.n ? ws->ncell : (int64_t)ws->cfg.n);
+// Pairs of a particle within the cutoff, itself apart: as told (sph_ws_tune),
+// else as if the particles filled the box.
+static double mean_pairs(const sph_ws* ws) {
+  const auto& c = ws->cfg;
+  if (ws->pairs > 0) return (double)ws->pairs / c.n - (c.mask_self ? 0.0 : 1.0);
+  double pairs = kBall[c.dim] * c.n;
+  for (int d = 0; d < c.dim; ++d) pairs *= (double)c.cutoff / (double)c.box[d];
+  return pairs;
 }
 
 // Exact lists: k_nl_tile's filter is the fast one's, and ordered (half) lists
@@ -1724,16 +1729,17 @@ static double occupied_cells(const sph_ws* ws) {
 static bool tiled(const sph_ws* ws) {
   const auto& c = ws->cfg;
   return fast_filter(c) && !c.ordered &&
-         tile_pays(c.dim, c.n, occupied_cells(ws), c.cell_size, c.cutoff, 15000.0);
+         tile_pays(c.dim, c.n, mean_pairs(ws), c.cell_size, c.cutoff, 15000.0);
 }
 // Skin lists, which the lanes build without a band: 2D 48,400 particles 22.7 and
 // 20.2 us, 67,600 (6,400 cells) 24.5 and 23.9, 78,400 (7,400) 25.3 and 26.1,
 // 136,900 30.7 and 33.2; Wendland C2 14,400 16.1 and 12.2, 57,600 17.2 and 19.9.
 static bool skin_tiled(const sph_ws* ws) {
   const auto& c = ws->cfg;
-  const auto& S = ws->sk;
-  const double occupied = occupied_cells(ws) * (double)S.ncell / (double)ws->ncell;
-  return tile_pays(c.dim, c.n, occupied, S.cell_size, c.cutoff + S.skin, 7000.0);
+  const float reach = c.cutoff + ws->sk.skin;
+  double pairs = mean_pairs(ws);
+  for (int d = 0; d < c.dim; ++d) pairs *= (double)reach / (double)c.cutoff;
+  return tile_pays(c.dim, c.n, pairs, ws->sk.cell_size, reach, 7000.0);
 }
 
 static unsigned build_grid(const sph_ws* ws, bool tile) {

@@ -66,9 +66,9 @@ struct sph_ws {
   // exact lists narrower than 3^d x cell capacity (sph_ws_tune "ell_overflow"):
   // a truncated sub-list raises SPH_NEIGHBOR_LIST_OVERFLOW
   int32_t ell_overflow = 0;
-  // cells of the grid that hold particles (sph_ws_tune "occupied_cells"; 0: not
-  // known), by which the pair build is chosen
-  int64_t occupied = 0;
+  // pairs of a list, about (sph_ws_tune "pairs"; 0: not known), by which the pair
+  // build is chosen
+  int64_t pairs = 0;
   int64_t bytes = 0;
   // binning scratch (shared by both banks)
   // The cell histogram: ncell, all zero between builds (the sort, or for skin

@@ -282,9 +282,9 @@ extern "C" int sph_ws_tune(sph_ws* ws, const char* key, int64_t value) {
     ws->ell_overflow = value ? 1 : 0;
     return SPH_OK;
   }
-  if (std::strcmp(key, "occupied_cells") == 0) {
-    if (value < 0) { set_error("sph_ws_tune: occupied_cells must be >= 0"); return SPH_ERR_ARG; }
-    ws->occupied = value;
+  if (std::strcmp(key, "pairs") == 0) {
+    if (value < 0) { set_error("sph_ws_tune: pairs must be >= 0"); return SPH_ERR_ARG; }
+    ws->pairs = value;
     return SPH_OK;
   }
   if (std::strcmp(key, "skin_rebuild") == 0) {

@@ -308,7 +308,7 @@ class _NeighborSearch:
         L = _lib.lib()
         st = _lib.stream()
         info = torch.zeros(8, dtype=torch.int64, device=dev)
-        cap, occupied = None, 0
+        cap = None
         if self.use_cells:
             # capacity estimate on the grid re-derived from the rounded cell size
             counts = torch.empty(int(np.prod(self.cps2.astype(np.int64))), dtype=torch.int32,
@@ -318,7 +318,6 @@ class _NeighborSearch:
             _lib.check(L.sph_nl_fill_max(dim, n, _lib.ptr(r), cs2, cp2, _lib.ptr(counts),
                                          _lib.ptr(info), st), "sph_nl_fill_max")
             max_fill = int(info[2])
-            occupied = int(torch.count_nonzero(counts))   # chooses the pair build
             cap = int(max_fill * self.capacity_multiplier) + int(extra_capacity)
             width = min(3 ** dim * max(cap, 1), n)
         else:
@@ -328,14 +327,15 @@ class _NeighborSearch:
         ws = _lib.Workspace(self._config(n, dim, cap, width))
         if ell_width is not None:
             ws.tune("ell_overflow", 1)
-        ws.tune("occupied_cells", occupied)
         ws.n, ws.dim, ws.cell_capacity = n, dim, cap
         ws.candidate_width = n * (3 ** dim) * cap if self.use_cells else n * n
         bank = 0
         ws.generation[bank] += 1
         _lib.check(L.sph_nl_build(ws.handle, bank, _lib.ptr(r), None, -1, _lib.ptr(info), st),
                    "sph_nl_build")
-        max_occ = self._max_occupancy(int(info[1]), ws, extra_capacity)
+        pairs = int(info[1])
+        ws.tune("pairs", pairs)   # chooses the pair build
+        max_occ = self._max_occupancy(pairs, ws, extra_capacity)
         _lib.check(L.sph_nl_finalize(ws.handle, max_occ, _lib.ptr(info), st), "sph_nl_finalize")
         self._scan_bits(ws, bank, info)
         self._enable_skin(ws, int(info[3]))

@@ -30,9 +30,10 @@ def test_exact_lists(dim, n, cells, part):
     nb = fn.allocate(t)
     idx, info = nb.idx, nb.info
     assert not bool(nb.did_buffer_overflow)
-    # as if the particles were alone in their cells, and as if ten (in 2D five) shared one
-    for told in (2 * n, n // (10 if dim == 3 else 5), 0):
-        nb.workspace.tune("occupied_cells", told)
+    # as if the particles had hardly a pair, a thousand, some fifteen or forty, and
+    # as if nothing were known of them
+    for told in (1, 1000 * n, (40 if dim == 3 else 15) * n, 0):
+        nb.workspace.tune("pairs", told)
         nb = nb.update(t)
         assert torch.equal(nb.info[:4], info[:4])
         assert torch.equal(nb.idx, idx), told
@@ -42,12 +43,12 @@ def test_exact_lists(dim, n, cells, part):
 def test_skin_lists(dim, side):
     """The last two have skin grids of four and three cells a side."""
     out = []
-    for told in (1 << 30, side ** dim // (20 if dim == 3 else 5)):
+    for told in (1, (80 if dim == 3 else 25) * side ** dim):
         dx = 2 * np.pi / side if dim == 3 else 1 / side
         cfg, state, nb, adv, *_ = _make("tgv", {"case": {"dim": dim, "dx": dx,
                                                          "r0_noise_factor": 0.1}})
         assert nb.workspace.skin_on
-        nb.workspace.tune("occupied_cells", told)
+        nb.workspace.tune("pairs", told)
         st, nb = adv(cfg.solver.dt, state, nb)
         out.append((nb.idx, nb.info[:4], st["r"], st["dudt"], st["rho"]))
     for a, b in zip(*out):
