@@ -1238,7 +1238,7 @@ __device__ __forceinline__ void nl_tile_body(ColdArgs* args, const int blk, cons
         // the grid) or not finite: the filter's bounds do not hold, and every
         // candidate of the piece is left to the exact one
         aa = ax = ay = az = 0.0f;
-        width = INFINITY;
+        width = 3.4e38f;
       }
       if (p >= np) aa = INFINITY;  // no particle: no hits
       int seg = 0;  // the last segment that starts before the candidates seen end
@@ -1317,51 +1317,80 @@ __device__ __forceinline__ void nl_tile_body(ColdArgs* args, const int blk, cons
             // one lane of hits (the compiler has no builtin for it)
             asm("v_writelane_b32 %0, %1, %2" : "+v"(hits) : "s"((int)__popcll(m[q])), "n"(q));
           }
-          if (__builtin_expect(__ballot(nearest < width || tops + hits > full) == 0ull, 1)) {
+          // the hits of each particle that `hit_of` gives as a lane mask, to the stage
+          const auto stage_hits = [&](auto&& hit_of) __attribute__((always_inline)) {
             for_blocks<0, P / 4>([&](auto qc) {
               constexpr int q0 = 4 * decltype(qc)::value;
               if (q0 >= np) return;  // uniform
 #pragma unroll
               for (int q = q0; q < q0 + 4; ++q) {
+                const mask_t mq = hit_of(q);
                 const unsigned k =
-                    __builtin_amdgcn_mbcnt_hi((unsigned)(m[q] >> 32),
-                                              __builtin_amdgcn_mbcnt_lo((unsigned)m[q], 0u));
+                    __builtin_amdgcn_mbcnt_hi((unsigned)(mq >> 32),
+                                              __builtin_amdgcn_mbcnt_lo((unsigned)mq, 0u));
                 const unsigned row = (unsigned)lane_i(tops, q);
                 Entry* const to = (Entry*)(uintptr_t)((k + row) << 1) + q * kRow;
-                if (__builtin_expect(__builtin_amdgcn_inverse_ballot_w64(m[q]), 1)) *to = entry;
+                if (__builtin_expect(__builtin_amdgcn_inverse_ballot_w64(mq), 1)) *to = entry;
               }
             });
             tops += hits;
+          };
+          if (__builtin_expect(__ballot(nearest < width || tops + hits > full) == 0ull, 1)) {
+            stage_hits([&](int q) { return m[q]; });
           } else {
-            // the exact filter, particle by particle; hits past the stage go
-            // straight to the buffer
+            // A lane's hits and its pairs within the band, a bit a particle; the
+            // exact filter decides the latter, one of each lane at a time.  On a
+            // lattice a chunk has some 40 such pairs, nearly every particle one:
+            // 1,000,000 on one took 1,503 us particle by particle (the lanes' build
+            // 902), so 825.
+            unsigned in = 0u, near = 0u;
+#pragma unroll
+            for (int q = 0; q < P; ++q) {
+              in |= d[q / 4][q % 4] < -width ? 1u << q : 0u;
+              near |= fabsf(d[q / 4][q % 4]) < width ? 1u << q : 0u;
+            }
             ColdArgs* const e = again(args);
             const float box[3] = {e->box[0], e->box[1], e->box[2]};
             const float half[3] = {e->half[0], e->half[1], e->half[2]};
             const float flo = e->lo, fhi = e->hi, csq = e->cutoff_sq;
-            const int lane_width = e->lane_width;
-            const int cj =
-                __shfl(lo, (int)(c >> kCandBits), 64) + (int)(c & ((1u << kCandBits) - 1u));
-#pragma unroll 1
-            for (int q = 0; q < np; ++q) {
-              const float4 pq = make_float4(lane_f(ps.x, q), lane_f(ps.y, q),
-                                            DIM == 3 ? lane_f(ps.z, q) : 0.0f, 0.0f);
+            while (__ballot(near != 0u)) {
+              const int q = near != 0u ? __ffs((int)near) - 1 : 0;
+              const float4 pq = make_float4(__shfl(ps.x, q, 64), __shfl(ps.y, q, 64),
+                                            DIM == 3 ? __shfl(ps.z, q, 64) : 0.0f, 0.0f);
               const float d2 = dist2<DIM>(pq.x - cix - pb.x, pq.y - ciy - pb.y,
                                           DIM == 3 ? pq.z - ciz - pb.z : 0.0f);
               const bool hit =
-                  valid && self != q &&
-                  (d2 < flo || (d2 < fhi && metric_sq_exact<DIM>(pq, pb, box, half) < csq));
-              const mask_t mq = __ballot(hit);
-              const int t = lane_i(tops, q);
-              const int k = t - (int)row0 +  // its number among the particle's hits
-                            (int)__builtin_amdgcn_mbcnt_hi(
-                                (unsigned)(mq >> 32),
-                                __builtin_amdgcn_mbcnt_lo((unsigned)mq, 0u));
-              if (hit && k < room)
-                *(Entry*)(uintptr_t)((k + row0 + q * kRow) << 1) = entry;
-              else if (hit && k / TPP < lane_width)
-                e->ell[((int64_t)(k % TPP) * lane_width + k / TPP) * e->npad + s0 + q] = cj;
-              tops = lane == q ? t + (int)__popcll(mq) : tops;
+                  d2 < flo || (d2 < fhi && metric_sq_exact<DIM>(pq, pb, box, half) < csq);
+              in |= hit && near != 0u ? 1u << q : 0u;
+              near &= near - 1u;
+            }
+#pragma unroll
+            for (int q = 0; q < P; ++q)
+              asm("v_writelane_b32 %0, %1, %2"
+                  : "+v"(hits) : "s"((int)__popcll(__ballot(in >> q & 1u))), "n"(q));
+            if (__ballot(tops + hits > full) == 0ull) {
+              stage_hits([&](int q) { return (mask_t)__ballot(in >> q & 1u); });
+            } else {
+              // hits past the stage go straight to the buffer
+              ColdArgs* const f = again(args);
+              const int lane_width = f->lane_width;
+              const int cj =
+                  __shfl(lo, (int)(c >> kCandBits), 64) + (int)(c & ((1u << kCandBits) - 1u));
+#pragma unroll 1
+              for (int q = 0; q < np; ++q) {
+                const bool hit = in >> q & 1u;
+                const mask_t mq = __ballot(hit);
+                const int t = lane_i(tops, q);
+                const int k = t - (int)row0 +  // its number among the particle's hits
+                              (int)__builtin_amdgcn_mbcnt_hi(
+                                  (unsigned)(mq >> 32),
+                                  __builtin_amdgcn_mbcnt_lo((unsigned)mq, 0u));
+                if (hit && k < room)
+                  *(Entry*)(uintptr_t)((k + row0 + q * kRow) << 1) = entry;
+                else if (hit && k / TPP < lane_width)
+                  f->ell[((int64_t)(k % TPP) * lane_width + k / TPP) * f->npad + s0 + q] = cj;
+                tops = lane == q ? t + (int)__popcll(mq) : tops;
+              }
             }
           }
         }
