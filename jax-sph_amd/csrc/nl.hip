@@ -1094,10 +1094,10 @@ __global__ __launch_bounds__(kBlock, ORDERED ? 1 : 6) void k_nl_build(BuildArgs 
 // mask's lower bits, and only the store to the stage runs for hits alone.
 // Squares within a band of the cutoff are decided by the filter of
 // nl_build_body.
-// Bound by the issue of instructions (vector 61%, scalar 64% of the cycles), 10
+// Bound by the issue of instructions (vector 78%, scalar 33% of the cycles), 10
 // for a particle and 64 candidates; a lane that tests candidates of its own
 // takes 9 per candidate and 25 per hit, in a loop as long as the wavefront's
-// longest.  Exact list of 1,000,000 3D particles 647 -> 421 us; tile_pays() has
+// longest.  Exact list of 1,000,000 3D particles 647 -> 398 us; tile_pays() has
 // the other sizes.
 // A stage entry is 16 bits (segment and offset in it, from which the sorted
 // index follows), so that 7 workgroups' stages fit a CU's LDS; entries past
@@ -1722,25 +1722,27 @@ static bool fast_filter(const sph_nl_config& c) {
 // 2D a piece's 64 candidates at a time are two chunks half full for each 9
 // particles, which pays until there are pieces for every SIMD: `most` cells.
 // Microseconds by the lanes' build and so, noisy lattices, exact lists:
-//   3D 256 particles, 0.3 a cell 39, 30; 9,000, 1 a cell 44, 34; 30,000, 1 a cell
-//   37, 38; 1.9 38, 30; 59 (245 pairs) 137, 124
-//   60,000, 1 a cell 43, 59; 3 48, 38; 27 93, 53; 45 (189 pairs) 144, 164
-//   300,000, 2.6 a cell 139, 142; 4.1 136, 101; 38 (157 pairs) 323, 184;
-//   51 (216 pairs) 411, 496
-//   2D 20,000, 2 a cell 18, 20; 3 19, 17; 32 (100 pairs) 56, 32
-//   60,000, 3 a cell 21, 25; 9 27, 20; 12 (37 pairs) 31, 23; 16 (51 pairs, 3,720
-//   cells) 38, 44; 20 (3,030 cells) 46, 35
-//   145,000, 4 a cell 25, 36; 9 (16,100 cells) 33, 33
-// 5,000 particles, half of them in one 3D cell (650 pairs) 175, 273.
+//   3D 9,000 particles, 0.5 a cell 41, 34; 30,000, 1 a cell 37, 40; 1.5 38, 35;
+//   59 (252 pairs) 137, 90
+//   60,000, 1 a cell 44, 63; 3 46, 39; 27 91, 51; 45 (194 pairs) 141, 135;
+//   60 (255 pairs) 122, 163
+//   300,000, 2.6 a cell 144, 150; 3.1 142, 128; 28 253, 136; 51 (215 pairs) 432,
+//   395; 1,000,000, 2.5 a cell 339, 417; 3 347, 367; 4 344, 305
+//   2D 20,000, 2 a cell 19, 20; 3 21, 16; 32 (99 pairs) 58, 25
+//   60,000, 3 a cell 21, 25; 4 (14,900 cells) 22, 21; 9 27, 20; 16 (49 pairs) 40, 35
+//   100,000, 5 a cell (19,900 cells) 26, 27; 7 30, 24; 16 (49 pairs, 6,200 cells)
+//   41, 46; 20 (62 pairs, 5,000 cells) 50, 42
+//   145,000, 4 a cell 25, 37; 9 (16,100 cells) 34, 30; 180,000, 9 (19,900) 36, 37
+// 5,000 particles, half of them in one 3D cell (650 pairs) 175, 218.
 static constexpr double kBall[] = {0.0, 2.0, 3.14, 4.19};
 static bool tile_pays(int dim, int64_t n, double pairs, const float* cell, float reach,
                       double most) {
   double held = pairs / kBall[dim];
   for (int d = 0; d < dim; ++d) held *= (double)cell[d] / (double)reach;
   if (dim == 3)
-    return held >= (n < 15000 ? 0.2 : n < 40000 ? 0.8 : 2.8) && pairs <= (n < 40000 ? 300.0 : 158.0);
+    return held >= (n < 15000 ? 0.2 : n < 40000 ? 0.8 : 2.8) && pairs <= (n < 40000 ? 400.0 : 220.0);
   const double cells = (double)n / held;
-  return held >= 2.5 && cells <= most && (pairs <= 43.0 || cells <= 3200.0);
+  return held >= 2.3 && cells <= most && (pairs <= 40.0 || cells <= 5200.0);
 }
 
 // Pairs of a particle within the cutoff, itself apart: as told (sph_ws_tune),
@@ -1758,17 +1760,17 @@ static double mean_pairs(const sph_ws* ws) {
 static bool tiled(const sph_ws* ws) {
   const auto& c = ws->cfg;
   return fast_filter(c) && !c.ordered &&
-         tile_pays(c.dim, c.n, mean_pairs(ws), c.cell_size, c.cutoff, 15000.0);
+         tile_pays(c.dim, c.n, mean_pairs(ws), c.cell_size, c.cutoff, 18000.0);
 }
-// Skin lists, which the lanes build without a band: 2D 48,400 particles 22.7 and
-// 20.2 us, 67,600 (6,400 cells) 24.5 and 23.9, 78,400 (7,400) 25.3 and 26.1,
-// 136,900 30.7 and 33.2; Wendland C2 14,400 16.1 and 12.2, 57,600 17.2 and 19.9.
+// Skin lists, which the lanes build without a band: 2D 48,400 particles 22.8 and
+// 17.0 us, 96,100 (9,100 cells) 26.0 and 24.4, 136,900 31.2 and 30.3; Wendland C2
+// 14,400 16.6 and 11.7, 57,600 (12,200 cells) 17.3 and 18.9.
 static bool skin_tiled(const sph_ws* ws) {
   const auto& c = ws->cfg;
   const float reach = c.cutoff + ws->sk.skin;
   double pairs = mean_pairs(ws);
   for (int d = 0; d < c.dim; ++d) pairs *= (double)reach / (double)c.cutoff;
-  return tile_pays(c.dim, c.n, pairs, ws->sk.cell_size, reach, 7000.0);
+  return tile_pays(c.dim, c.n, pairs, ws->sk.cell_size, reach, 10000.0);
 }
 
 static unsigned build_grid(const sph_ws* ws, bool tile) {
