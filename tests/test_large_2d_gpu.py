@@ -1,6 +1,6 @@
-"""2D sets beyond 150,000 particles, whose builds compare candidate by candidate:
-the exact list of a lattice with pairs exactly at the cutoff, and the skin list
-of a few steps, against the oracle's per-step search."""
+"""Large 2D sets, by either pair build: the exact list of a lattice with pairs
+exactly at the cutoff, and the skin list of a few steps, against the oracle's
+per-step search."""
 import numpy as np
 import pytest
 import torch
@@ -24,18 +24,26 @@ def test_lattice_pairs_at_the_cutoff(mask_self):
     disp, _ = space.periodic(side=np.ones(2))
     fn = partition.neighbor_list(disp, np.ones(2), r_cutoff=3 / side, mask_self=mask_self,
                                  format=partition.Sparse)
-    nb = fn.allocate(torch.tensor(r, device="cuda"))
+    t = torch.tensor(r, device="cuda")
+    nb = fn.allocate(t)
     want = nlo.sorted_pairs(nlo.NeighborSearch(np.ones(2), 3 / side,
                                                mask_self=mask_self).allocate(r).idx, n)
     assert np.array_equal(nlo.sorted_pairs(nb.idx.cpu().numpy(), n), want)
+    # as if a particle had 28 pairs, and hardly any: one build and the other
+    for told in (28 * n, 1):
+        nb.workspace.tune("pairs", told)
+        nb = nb.update(t)
+        assert np.array_equal(nlo.sorted_pairs(nb.idx.cpu().numpy(), n), want)
 
 
-def test_skin_list():
+@pytest.mark.parametrize("told", [90 * 160000, 1])
+def test_skin_list(told):
     cfg, state, nb, adv, R, fn, *_ = _make("tgv", {"case": {"dim": 2, "dx": 1 / 400,
                                                              "r0_noise_factor": 0.1}})
     assert nb.workspace.skin_on and nb.workspace.n == 160000
     ref_nb = R.ns.allocate(state["r"].cpu().numpy())
     st = state
+    nb.workspace.tune("pairs", told)
     for k in range(3):
         if k == 2:
             nb.workspace.tune("skin_rebuild", 1)
