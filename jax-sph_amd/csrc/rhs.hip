@@ -192,12 +192,12 @@ SPH_SWEEP_KERNELS(k_renorm, renorm_run, (int DIM, int KIND), (DIM, KIND), 8)
 // EXTRAS: artificial viscosity and heat conduction are compiled in (otherwise
 // the sweep cannot issue the extra per-pair loads they need).
 template <int DIM, int KIND, int SOLVER, bool TVF, bool EXTRAS>
-__device__ __forceinline__ void force_run(const SweepArgs& a, const int blk) {
+__device__ __forceinline__ void force_run(const SweepArgs& a, const int blk, const bool tail) {
   constexpr int TPP = tpp_of(DIM);
   const int tid = blk * blockDim.x + threadIdx.x;
   const int s = tid / TPP, h = tid % TPP;
   if (s >= a.n) {  // whole lane groups leave together
-    if (tail_block(a)) reduce_parts_body<kB>(a.tail);
+    if (tail && blockIdx.x == 0) reduce_parts_body<kB>(a.tail);
     return;
   }
   const sph_solver_params& p = a.prm;
@@ -368,9 +368,9 @@ __device__ __forceinline__ void force_run(const SweepArgs& a, const int blk) {
   if (o.T) o.T[i] = Ti;
   if (o.dTdt) o.dTdt[i] = heat ? dT : (a.in.dTdt ? a.in.dTdt[i] : 0.0f);
 }
-SPH_SWEEP_KERNELS(k_force, force_run, (int DIM, int KIND, int SOLVER, bool TVF, bool EXTRAS),
-                  (DIM, KIND, SOLVER, TVF, EXTRAS),
-                  (SOLVER == 0 && !EXTRAS && KIND >= 0 ? 8 : 1))
+SPH_TAIL_SWEEP_KERNELS(k_force, force_run, (int DIM, int KIND, int SOLVER, bool TVF, bool EXTRAS),
+                       (DIM, KIND, SOLVER, TVF, EXTRAS),
+                       (SOLVER == 0 && !EXTRAS && KIND >= 0 ? 8 : 1))
 
 // ------------------------------------------------------------- integrate
 // si_euler kick + transport velocity + drift + periodic wrap (integrator.py:26-30)

@@ -195,24 +195,12 @@ struct SweepArgs {
   int64_t* info;  // non-null: the density sweep counts pairs (per-workgroup partials in part)
   int64_t* part;  // [2 * gridDim.x] pairs and largest list of each workgroup
   int remap;      // XCD-contiguous block order (grid a multiple of 8)
-  // tail.part non-null: the launch's first workgroup reduces the partials of
-  // an earlier launch (a launch of its own costs the stream 4-5 us, and nothing
-  // of this sweep reads the result); kTailBlocks more than the sweep's own
+  // density and force sweeps, tail.part non-null: the launch's first workgroup
+  // reduces the partials of an earlier launch (a launch of its own costs the
+  // stream 4-5 us, and nothing of this sweep reads the result); kTailBlocks more
+  // than the sweep's own
   Reduce tail;
 };
-
-// The workgroup that reduces for an earlier launch.  The sweeps look for it
-// where threads without a particle leave anyway: a branch before the sweep
-// costs its loop registers (the 3D standard force with transport velocity,
-// which fills its 64, went to scratch memory: 1,566 us at 128^3, without the
-// branch 1,557; the delta-SPH force with artificial viscosity lost a wavefront
-// a SIMD: 178 us at 64^3, without 170).
-__device__ __forceinline__ bool tail_block(const SweepArgs& a) {
-  return a.tail.part != nullptr && blockIdx.x == 0;
-}
-__device__ __forceinline__ int sweep_block(const SweepArgs& a) {
-  return sweep_block_of(blockIdx.x, gridDim.x, a.tail.part != nullptr, a.remap);
-}
 
 // Pair (sweep centre s, listed j) of the neighbour set: the reference predicate
 // metric_sq(r_s, r_j) < cutoff^2 with s in the sender role, as in the build.
@@ -369,14 +357,31 @@ __global__ void k_gather_state(SweepArgs a, const float* __restrict__ r, const f
 #define SPH_SWEEP_KERNELS(NAME, RUN, TPARAMS, TARGS, MINW)                                \
   template <SPH_UNPAREN TPARAMS>                                                          \
   __global__ __launch_bounds__(kB, MINW) void NAME(SweepArgs a) {                         \
-    RUN<SPH_UNPAREN TARGS>(a, sweep_block(a));                                            \
+    RUN<SPH_UNPAREN TARGS>(a, logical_block(a.remap));                                    \
   }                                                                                       \
+  SPH_ENSEMBLE_KERNEL(NAME, RUN, TPARAMS, TARGS, MINW, (t[m.sim], m.blk))
+// The same around RUN<TARGS>(args, blk, tail) for sweeps that may have a tail:
+// tail is set in the workgroups in front.  The body looks for it where threads
+// without a particle leave anyway: a branch before the sweep costs its loop
+// registers (the 3D standard force with transport velocity, which fills its 64,
+// went to scratch memory: 1,566 us at 128^3, without the branch 1,557; the
+// delta-SPH force with artificial viscosity lost a wavefront a SIMD: 178 us at
+// 64^3, without 170).
+#define SPH_TAIL_SWEEP_KERNELS(NAME, RUN, TPARAMS, TARGS, MINW)                           \
+  template <SPH_UNPAREN TPARAMS>                                                          \
+  __global__ __launch_bounds__(kB, MINW) void NAME(SweepArgs a) {                         \
+    const bool ride = a.tail.part != nullptr;                                             \
+    RUN<SPH_UNPAREN TARGS>(a, sweep_block_of(blockIdx.x, gridDim.x, ride, a.remap),       \
+                           ride && (int)blockIdx.x < kTailBlocks);                        \
+  }                                                                                       \
+  SPH_ENSEMBLE_KERNEL(NAME, RUN, TPARAMS, TARGS, MINW, (t[m.sim], m.blk, false))
+#define SPH_ENSEMBLE_KERNEL(NAME, RUN, TPARAMS, TARGS, MINW, ARGS)                        \
   template <SPH_UNPAREN TPARAMS>                                                          \
   __global__ __launch_bounds__(kB, MINW) void NAME##_ens(const SweepArgs* __restrict__ t, \
-                                                         const EnsBlock* __restrict__ map) { \
+                                                         const EnsBlock* __restrict__ map) {\
     const EnsBlock m = map[blockIdx.x];                                                   \
     if (m.sim < 0) return;                                                                \
-    RUN<SPH_UNPAREN TARGS>(t[m.sim], m.blk);                                              \
+    RUN<SPH_UNPAREN TARGS> ARGS;                                                          \
   }
 
 // Arguments of one ensemble member's gather: the sweep arguments plus the
@@ -542,8 +547,8 @@ __device__ __forceinline__ int density_of(const SweepArgs& a, const int s, const
 // blk: the workgroup's block within this list's grid; it also indexes the
 // workgroup's partials.
 template <int DIM, int KIND, int MODE>
-__device__ __forceinline__ void density_run(const SweepArgs& a, const int blk) {
-  if (a.tail.part && (int)blockIdx.x < kTailBlocks) {
+__device__ __forceinline__ void density_run(const SweepArgs& a, const int blk, const bool tail) {
+  if (tail) {
     if (blockIdx.x == 0) reduce_parts_body<kB>(a.tail);
     return;
   }
@@ -578,7 +583,8 @@ __device__ __forceinline__ void density_run(const SweepArgs& a, const int blk) {
   }
 }
 
-SPH_SWEEP_KERNELS(k_density, density_run, (int DIM, int KIND, int MODE), (DIM, KIND, MODE), 8)
+SPH_TAIL_SWEEP_KERNELS(k_density, density_run, (int DIM, int KIND, int MODE), (DIM, KIND, MODE),
+                       8)
 
 // ------------------------------------------------------------- walls
 // MODE 0: generalized wall BC of the SPH solver (solver.py:431-530)
