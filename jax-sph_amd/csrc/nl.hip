@@ -1131,7 +1131,7 @@ __device__ __forceinline__ ColdArgs* again(ColdArgs* a) {
 }
 
 // R: consecutive sorted particles of a workgroup, which takes the pieces that
-// start there (tile_range, or what the caller's grid makes of it).
+// start there (tile_pays, or what the caller's grid makes of it).
 template <int DIM, int TPP>
 __device__ __forceinline__ void nl_tile_body(ColdArgs* args, const int blk, const int R) {
   constexpr int W = kBlock / 64, S = tile_stage(DIM), P = tile_rows(DIM);
@@ -1734,15 +1734,26 @@ static bool fast_filter(const sph_nl_config& c) {
 //   41, 46; 20 (62 pairs, 5,000 cells) 50, 42
 //   145,000, 4 a cell 25, 37; 9 (16,100 cells) 34, 30; 180,000, 9 (19,900) 36, 37
 // 5,000 particles, half of them in one 3D cell (650 pairs) 175, 218.
+// Returns 0, or the consecutive particles a workgroup takes.  Its four wavefronts
+// take in turn the pieces that start there, and it lasts as long as the one with
+// the most: 32 leaves most with one; 48 where about a piece each still covers
+// them and every SIMD has work (27 a cell 21,952 particles 32 and 42 us, 97,336
+// 69 and 66, 262,144 147 and 127, 2,097,152 1,024 and 834, skin lists at 35 a cell
+// 1,199 and 996; 18 a cell 262,144 74 and 79, 2,097,152 503 and 521).
 static constexpr double kBall[] = {0.0, 2.0, 3.14, 4.19};
-static bool tile_pays(int dim, int64_t n, double pairs, const float* cell, float reach,
-                      double most) {
+static int tile_pays(int dim, int64_t n, double pairs, const float* cell, float reach,
+                     double most) {
   double held = pairs / kBall[dim];
   for (int d = 0; d < dim; ++d) held *= (double)cell[d] / (double)reach;
-  if (dim == 3)
-    return held >= (n < 15000 ? 0.2 : n < 40000 ? 0.8 : 2.8) && pairs <= (n < 40000 ? 400.0 : 220.0);
+  if (dim == 3) {
+    if (held < (n < 15000 ? 0.2 : n < 40000 ? 0.8 : 2.8) || pairs > (n < 40000 ? 400.0 : 220.0))
+      return 0;
+    constexpr int kMore = 48;
+    const double pieces = std::ceil(held / tile_rows(3)) / held;  // a particle
+    return n >= 80000 && kMore * pieces <= 1.15 * (kBlock / 64) ? kMore : kTileRange;
+  }
   const double cells = (double)n / held;
-  return held >= 2.3 && cells <= most && (pairs <= 40.0 || cells <= 5200.0);
+  return held >= 2.3 && cells <= most && (pairs <= 40.0 || cells <= 5200.0) ? kTileRange : 0;
 }
 
 // Pairs of a particle within the cutoff, itself apart: as told (sph_ws_tune),
@@ -1757,15 +1768,15 @@ static double mean_pairs(const sph_ws* ws) {
 
 // Exact lists: k_nl_tile's filter is the fast one's, and ordered (half) lists
 // compare ids candidate by candidate.
-static bool tiled(const sph_ws* ws) {
+static int tile_range(const sph_ws* ws) {
   const auto& c = ws->cfg;
-  return fast_filter(c) && !c.ordered &&
-         tile_pays(c.dim, c.n, mean_pairs(ws), c.cell_size, c.cutoff, 18000.0);
+  if (!fast_filter(c) || c.ordered) return 0;
+  return tile_pays(c.dim, c.n, mean_pairs(ws), c.cell_size, c.cutoff, 18000.0);
 }
 // Skin lists, which the lanes build without a band: 2D 48,400 particles 22.8 and
 // 17.0 us, 96,100 (9,100 cells) 26.0 and 24.4, 136,900 31.2 and 30.3; Wendland C2
 // 14,400 16.6 and 11.7, 57,600 (12,200 cells) 17.3 and 18.9.
-static bool skin_tiled(const sph_ws* ws) {
+static int skin_tile_range(const sph_ws* ws) {
   const auto& c = ws->cfg;
   const float reach = c.cutoff + ws->sk.skin;
   double pairs = mean_pairs(ws);
@@ -1773,10 +1784,9 @@ static bool skin_tiled(const sph_ws* ws) {
   return tile_pays(c.dim, c.n, pairs, ws->sk.cell_size, reach, 10000.0);
 }
 
-static unsigned build_grid(const sph_ws* ws, bool tile) {
+static unsigned build_grid(const sph_ws* ws, int range) {
   const auto& c = ws->cfg;
-  const int64_t blocks = tile ? cdiv(c.n, tile_range(c.dim, c.n))
-                              : cdiv((int64_t)c.n * ws->tpp, kBlock);
+  const int64_t blocks = range ? cdiv(c.n, range) : cdiv((int64_t)c.n * ws->tpp, kBlock);
   return xcd_grid(blocks, ws->xcd_remap);
 }
 
@@ -1807,23 +1817,23 @@ int build_pairs(sph_ws* ws, int bank, int64_t* info, hipStream_t st) {
   a.gate = nullptr;
   a.remap = ws->xcd_remap;
   a.fast = fast_filter(c);
-  a.range = tile_range(c.dim, c.n);
+  a.range = tile_range(ws);
   cut_band(c, &a.lo, &a.hi);
   a.tile = tile_band(a.box, a.g.cs, c.dim, c.cutoff, a.cutoff_sq);
   constexpr int T2 = tpp_of(2), T3 = tpp_of(3);
-  const bool d2 = c.dim == 2, tile = tiled(ws);
+  const bool d2 = c.dim == 2;
   const auto kernel =
-      tile        ? (d2 ? k_nl_tile<2, T2> : k_nl_tile<3, T3>)
+      a.range     ? (d2 ? k_nl_tile<2, T2> : k_nl_tile<3, T3>)
       : c.ordered ? (d2 ? k_nl_build<2, T2, true, true> : k_nl_build<3, T3, true, true>)
                   : (d2 ? k_nl_build<2, T2, false, true> : k_nl_build<3, T3, false, true>);
-  SPH_LAUNCH(ws, "nl_build", st, (kernel<<<build_grid(ws, tile), kBlock, 0, st>>>(a)));
+  SPH_LAUNCH(ws, "nl_build", st, (kernel<<<build_grid(ws, a.range), kBlock, 0, st>>>(a)));
   return SPH_OK;
 }
 
 // What an exact build leaves to reduce: occupancy info[1], largest list
 // info[3], and the overflow bit when max_occupancy >= 0.
 Reduce build_tail(sph_ws* ws, int64_t max_occupancy, int64_t* info) {
-  const int blocks = (int)build_grid(ws, tiled(ws));
+  const int blocks = (int)build_grid(ws, tile_range(ws));
   return Reduce{ws->part_build, blocks, &info[1], &info[3], info, max_occupancy, nullptr, nullptr};
 }
 
@@ -1941,7 +1951,7 @@ static BuildArgs skin_build_args(sph_ws* ws, int64_t* info) {
   }
   a.cutoff_sq = S.reach_sq;
   a.fast = 1;
-  a.range = tile_range(c.dim, c.n);
+  a.range = skin_tile_range(ws);
   a.lo = a.hi = S.reach_sq;
   a.tile = tile_band(a.box, a.g.cs, c.dim, c.cutoff + S.skin, a.cutoff_sq);
   a.n = c.n;
@@ -1960,17 +1970,18 @@ int skin_build(sph_ws* ws, int64_t* info, hipStream_t st) {
   auto& S = ws->sk;
   const BuildArgs a = skin_build_args(ws, info);
   constexpr int T2 = tpp_of(2), T3 = tpp_of(3);
-  const bool d2 = c.dim == 2, tile = skin_tiled(ws);
-  const auto kernel = tile ? (d2 ? k_nl_tile<2, T2> : k_nl_tile<3, T3>)
-                           : (d2 ? k_nl_build<2, T2, false, false> : k_nl_build<3, T3, false, false>);
-  SPH_LAUNCH(ws, "skin_build", st, (kernel<<<build_grid(ws, tile), kBlock, 0, st>>>(a)));
+  const bool d2 = c.dim == 2;
+  const auto kernel =
+      a.range ? (d2 ? k_nl_tile<2, T2> : k_nl_tile<3, T3>)
+              : (d2 ? k_nl_build<2, T2, false, false> : k_nl_build<3, T3, false, false>);
+  SPH_LAUNCH(ws, "skin_build", st, (kernel<<<build_grid(ws, a.range), kBlock, 0, st>>>(a)));
   return SPH_OK;
 }
 
 // What a skin build leaves to reduce: the largest list of one particle ->
 // info[7] (only on a rebuild).
 Reduce skin_build_tail(sph_ws* ws, int64_t* info) {
-  const int blocks = (int)build_grid(ws, skin_tiled(ws));
+  const int blocks = (int)build_grid(ws, skin_tile_range(ws));
   return Reduce{ws->part_build, blocks, nullptr, &info[7], info, -1, ws->sk.flag, nullptr};
 }
 
@@ -2090,7 +2101,7 @@ __global__ __launch_bounds__(256) void k_cell_sort_ens(const EnsBin* __restrict_
 }
 
 // The members of a 2D ensemble are many particles together, where the lanes'
-// build is the faster one (see skin_tiled()).
+// build is the faster one (see skin_tile_range()).
 template <int DIM, int TPP>
 __global__ __launch_bounds__(kBlock, 6) void k_nl_build_ens(const BuildArgs* __restrict__ t,
                                                             const EnsBlock* __restrict__ map) {

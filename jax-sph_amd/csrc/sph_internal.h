@@ -34,14 +34,9 @@ __host__ __device__ constexpr int tpp_of(int dim) { return dim == 3 ? 4 : 2; }
 // up to 31 TPP entries past a cell range, without clamping each one.
 constexpr int kSkinPosPad = 128;
 
-// Consecutive sorted particles of a workgroup of the matrix-core pair build,
-// whose four wavefronts take in turn the pieces (up to 12 or 16 particles of
-// one cell) that start there.  A workgroup lasts as long as the wavefront with
-// the most pieces: 32 leaves most with one (3D 28^3 particles 34 us; with 48,
-// 45 us), 48 fewer of them idle where every SIMD has work (64^3: 154 and 128).
-__host__ __device__ constexpr int tile_range(int dim, int64_t n) {
-  return dim == 2 || n < 80000 ? 32 : 48;
-}
+// Consecutive sorted particles of a workgroup of the matrix-core pair build, at
+// the least.
+constexpr int kTileRange = 32;
 
 struct ProfEntry {
   const char* name;

@@ -118,10 +118,10 @@ extern "C" int sph_ws_create(const sph_nl_config* cfg, sph_ws** out) {
   A(ws->off64, N + 1);
   A(ws->scan_tmp, 1024);
   A(ws->cnt_id, N);
-  // workgroups of the widest launch (npad * tpp lanes of 256, or tile_range
+  // workgroups of the widest launch (npad * tpp lanes of 256, or kTileRange
   // particles each; rounded to 8 XCDs)
   const int64_t sweep_blocks = (npad * ws->tpp + 255) / 256;
-  const int64_t range = tile_range(cfg->dim, N), tile_blocks = (N + range - 1) / range;
+  const int64_t tile_blocks = (N + kTileRange - 1) / kTileRange;
   ws->part_blocks =
       (int32_t)(((sweep_blocks > tile_blocks ? sweep_blocks : tile_blocks) + 7) / 8 * 8);
   A(ws->part_build, 2 * (int64_t)ws->part_blocks);
