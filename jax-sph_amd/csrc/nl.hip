@@ -1736,10 +1736,11 @@ static bool fast_filter(const sph_nl_config& c) {
 // 5,000 particles, half of them in one 3D cell (650 pairs) 175, 218.
 // Returns 0, or the consecutive particles a workgroup takes.  Its four wavefronts
 // take in turn the pieces that start there, and it lasts as long as the one with
-// the most: 32 leaves most with one; 48 where about a piece each still covers
-// them and every SIMD has work (27 a cell 21,952 particles 32 and 42 us, 97,336
-// 69 and 66, 262,144 147 and 127, 2,097,152 1,024 and 834, skin lists at 35 a cell
-// 1,199 and 996; 18 a cell 262,144 74 and 79, 2,097,152 503 and 521).
+// the most: 32 leaves most with one; 48, fewer workgroups, is the faster where
+// about a piece each still covers them and every SIMD has work (27 a cell 21,952
+// particles 32 and 42 us, 97,336 69 and 66, 262,144 147 and 127, 2,097,152 1,024
+// and 834, skin lists at 35 a cell 1,199 and 996; 8 a cell 262,144 74 and 79,
+// 2,097,152 503 and 521, skin lists at 10 a cell 81 and 83, 535 and 514).
 static constexpr double kBall[] = {0.0, 2.0, 3.14, 4.19};
 static int tile_pays(int dim, int64_t n, double pairs, const float* cell, float reach,
                      double most) {
@@ -1749,8 +1750,9 @@ static int tile_pays(int dim, int64_t n, double pairs, const float* cell, float 
     if (held < (n < 15000 ? 0.2 : n < 40000 ? 0.8 : 2.8) || pairs > (n < 40000 ? 400.0 : 220.0))
       return 0;
     constexpr int kMore = 48;
-    const double pieces = std::ceil(held / tile_rows(3)) / held;  // a particle
-    return n >= 80000 && kMore * pieces <= 1.15 * (kBlock / 64) ? kMore : kTileRange;
+    const double cell_holds = held * (pairs + 1.0) / pairs;  // the particle itself too
+    const double pieces = kMore * std::ceil(cell_holds / tile_rows(3)) / cell_holds;
+    return n >= 80000 && pieces <= 5.5 ? kMore : kTileRange;
   }
   const double cells = (double)n / held;
   return held >= 2.3 && cells <= most && (pairs <= 40.0 || cells <= 5200.0) ? kTileRange : 0;
