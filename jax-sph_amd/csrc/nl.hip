@@ -1094,7 +1094,7 @@ __global__ __launch_bounds__(kBlock, ORDERED ? 1 : 6) void k_nl_build(BuildArgs 
 // mask's lower bits, and only the store to the stage runs for hits alone.
 // Squares within a band of the cutoff are decided by the filter of
 // nl_build_body.
-// Bound by the issue of instructions (vector 82%, scalar 34% of the cycles, the
+// Bound by the issue of instructions (vector 83%, scalar 35% of the cycles, the
 // matrix cores busy in 12%), 10 for a particle and 64 candidates; a lane that
 // tests candidates of its own takes 9 per candidate and 25 per hit, in a loop as
 // long as the wavefront's longest.  Exact list of 1,000,000 3D particles
